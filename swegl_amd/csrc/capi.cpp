@@ -1263,7 +1263,7 @@ static int build_wave(swegl_ctx *c, Lane &L, const std::vector<JobIn> &jobs, Wav
     // keep theirs
     W.fixed = false;
     W.fixed_total = 0;
-    if ((!arena || L.own_views) && !W.layers && W.tiles && tris_total < 0x80000000ull) {   // (SW_BIN_CHECK: top bit)
+    if ((!arena || L.own_views) && !W.layers && W.tiles && tris_total < 0x40000000ull) {   // (SW_BIN_CHECK, SW_BIN_LARGE: top bits)
         uint64_t total = 0;
         for (JobDev &J : W.jd) {
             const uint64_t tiles = (uint64_t)J.tiles_x * J.tiles_y;

@@ -69,46 +69,56 @@ SW_HD f3 neg(f3 a) { return {-a.x, -a.y, -a.z}; }
 // vector_t::dot (points.hpp:93): (xx + yy) + zz
 SW_HD float dot(f3 a, f3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
 
-// Correctly rounded a / b for several numerators over one denominator b,
-// for callers that know 1 <= b <= 2^20 and a == 0 or 2^-60 <= |a| <= 2^60.
-// The compiler expands each IEEE '/' into: v_div_scale of a and b, r =
-// rcp(b) refined by one fma step, q = a*r, two fma residual corrections
-// (the last through v_div_fmas), then v_div_fixup.  In that range the
-// scaling and the fixup are identities, so the refined reciprocal depends
-// on b alone and is computed once; each quotient then takes five
-// instructions and equals '/' bit for bit (a zero numerator keeps its
-// signed zero a*r).
+// ------------------------- exact reciprocal, quotient and square root
+// The compiler's IEEE '/' and sqrtf scale their operands so that they hold
+// over the whole float range, at 11 and 15 instructions (and wait states
+// around v_div_fmas).  Where the operands are known to lie well inside the
+// range the scaling is the identity, and shorter forms round the same way:
+//  - rcp_rn: v_rcp_f32 and one Newton step equal 1 / b, and sqrt_rn equals
+//    sqrtf, for every float from 2^-96 to 2^96 (compared on the device over
+//    all 1.6e9 of them);
+//  - div_rn: with r = rcp_rn(b), one residual correction equals a / b for
+//    every pair of significands (all 2^46 compared on the device through the
+//    exact residual) while a and the quotient stay within 2^-90 .. 2^120 and
+//    b within 2^-47 .. 2^47 (the residual is then exact); a positive zero a
+//    gives a positive zero.
+// A GPU test repeats the unary comparisons in full and samples the quotients.
+SW_D float rcp_rn(float b)
+{
+    const float r0 = __builtin_amdgcn_rcpf(b);
+    return __builtin_fmaf(__builtin_fmaf(-b, r0, 1.0f), r0, r0);
+}
+SW_D float div_rn(float a, float b, float r)
+{
+    const float q = a * r;
+    return __builtin_fmaf(__builtin_fmaf(-b, q, a), r, q);
+}
+SW_D float sqrt_rn(float x)
+{
+    const float y = __builtin_amdgcn_rsqf(x), g = x * y, h = 0.5f * y;
+    return __builtin_fmaf(__builtin_fmaf(-g, g, x), h, g);
+}
+
+// Several quotients over one denominator, in div_rn's range.
 struct FDiv {
     float b, r;
-    SW_D explicit FDiv(float den) : b(den)
-    {
-        const float r0 = __builtin_amdgcn_rcpf(den);
-        r = __builtin_fmaf(__builtin_fmaf(-den, r0, 1.0f), r0, r0);
-    }
-    SW_D float operator()(float a) const { return a == 0.0f ? a * r : nonzero(a); }
-    // the quotient of a nonzero numerator in the range above
-    SW_D float nonzero(float a) const
-    {
-        const float q0 = a * r;
-        float q = __builtin_fmaf(__builtin_fmaf(-b, q0, a), r, q0);
-        return __builtin_fmaf(__builtin_fmaf(-b, q, a), r, q);
-    }
+    SW_D explicit FDiv(float den) : b(den), r(rcp_rn(den)) {}
+    SW_D float operator()(float a) const { return div_rn(a, b, r); }
 };
 
-// vector_t::normalize (points.hpp:80-90).  When every component is at
-// least 2^-60 in magnitude and the length l at most 2^40, the compiler's
-// expansion of each x / l scales nothing (l and 1/l normal, the numerator's
-// exponent within 96 of l's and above 2^-103, the quotient at least 2^-100),
-// so the three quotients share l's refined reciprocal (FDiv's steps, here
-// without its zero case); otherwise the plain divisions.
-SW_D f3 normalize(f3 a)
+// vector_t::normalize (points.hpp:80-90).  With every component at least
+// 2^-40 in magnitude and the squared length at most 2^80, the square root
+// and the three quotients take the short forms above and share the length's
+// reciprocal; otherwise sqrtf and the plain divisions.  `s` is the squared
+// length as the reference sums it.
+SW_D f3 normalize_s(f3 a, float s)
 {
-    float l = sqrtf(a.x * a.x + a.y * a.y + a.z * a.z);
     const float m = fminf(fabsf(a.x), fminf(fabsf(a.y), fabsf(a.z)));
-    if (m >= 0x1p-60f && l <= 0x1p40f) {
-        const FDiv by(l);
-        return {by.nonzero(a.x), by.nonzero(a.y), by.nonzero(a.z)};
+    if (m >= 0x1p-40f && s <= 0x1p80f) {
+        const float l = sqrt_rn(s), r = rcp_rn(l);
+        return {div_rn(a.x, l, r), div_rn(a.y, l, r), div_rn(a.z, l, r)};
     }
+    const float l = sqrtf(s);
     if (l != 0) {
         a.x /= l;
         a.y /= l;
@@ -116,6 +126,7 @@ SW_D f3 normalize(f3 a)
     }
     return a;
 }
+SW_D f3 normalize(f3 a) { return normalize_s(a, a.x * a.x + a.y * a.y + a.z * a.z); }
 // cross() builds a normal_t, which normalises (points.cpp:32-37); only the
 // sign of the normalised z component is ever read on the path:
 // sign(normalize(cross(l, r)).z) compared with 0 (dir = +1: > 0, -1: < 0)

@@ -159,8 +159,11 @@ struct BatchDev {
 #define SW_CTR_OVERFLOW (SW_CTR_TOTAL + 32)   // nonzero: a tile passed tile_cap
 // A fixed-layout bin entry with this bit set names a triangle that failed its
 // own visibility test: it is drawn only if other triangles marked all three
-// of its vertices, which the raster looks up (a job holds < 2^31 triangles)
+// of its vertices, which the raster looks up
 #define SW_BIN_CHECK 0x80000000u
+// and one with this bit set a triangle whose bounding box holds more than
+// SW_LANE_PIXELS pixels (a job of the fixed layout holds < 2^30 triangles)
+#define SW_BIN_LARGE 0x40000000u
 #define SW_CTR_TICKETS (SW_CTR_TOTAL + 64)
 #define SW_CTR_BIG0 (SW_CTR_TICKETS + 32 * (SW_TICKET_GROUPS + 1))
 // statistic indices within a slot

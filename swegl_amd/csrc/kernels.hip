@@ -167,7 +167,9 @@ __global__ __launch_bounds__(256) void k_vertex(BatchDev B, uint32_t w0, uint32_
         return;
     const float4 w4 = ro4(J.world, i);
     const f3 f = world_to_frustum(J.V, f3{w4.x, w4.y, w4.z});
-    J.ndc[i] = make_float4(f.x, f.y, f.z, 0.0f);
+    // 1 / z: the interpolators' start value (interpolator.hpp:58-62), which
+    // every setup of a triangle with this vertex would divide out again
+    J.ndc[i] = make_float4(f.x, f.y, f.z, 1.0f / f.z);
     J.yes[i] = 0;
 }
 
@@ -410,6 +412,14 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v)
     return v;
 }
 
+__device__ __forceinline__ uint32_t wave_sum(uint32_t v)
+{
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+        v += __shfl_xor(v, o);
+    return v;
+}
+
 // Claim order of the raster's tiles: largest bin counts first (a counting
 // sort on a logarithmic bucket of the count, four buckets per power of
 // two), so that the costliest tiles start first and the last ones to start
@@ -537,6 +547,10 @@ __device__ void order_tiles(const BatchDev &B)
 }
 
 // ------------------------------------------------------------- k_front
+// Tiles of more than 256 entries: the most pixels that one lane replays on its
+// own; smallest chunk (pixels) of a listed triangle.
+#define SW_LANE_PIXELS 96
+#define SW_CHUNK_PIXELS 8
 // Per triangle, in one pass: the visibility marks (renderer.cpp:83-185: a
 // triangle passing the frustum test and double-sided or front-facing marks
 // its three vertices), its tile rectangle (conservative but never too small:
@@ -558,6 +572,7 @@ __global__ __launch_bounds__(256) void k_front(BatchDev B, const JobDev *__restr
     uint32_t big = 0;
     int ntiles = 0, tx0 = 0, tx1 = 0, ty0 = 0;
     bool self_marked = false;   // marked its own vertices: drawn whatever other triangles do
+    bool large = false;         // may cover more than SW_LANE_PIXELS pixels of a tile
     if (t < J.n_tris) {
         const uint32_t i0 = ro(J.tri)[3 * t], i1 = ro(J.tri)[3 * t + 1], i2 = ro(J.tri)[3 * t + 2];
         const f3 a = ld3(J.ndc, i0), b = ld3(J.ndc, i1), c = ld3(J.ndc, i2);
@@ -579,6 +594,7 @@ __global__ __launch_bounds__(256) void k_front(BatchDev B, const JobDev *__restr
         if (have) {
             int ty1;
             r = tile_rect(J, E, tx0, tx1, ty0, ty1);
+            large = (int64_t)(E.x1 - E.x0) * (E.y1 - E.y0) > SW_LANE_PIXELS;
             ntiles = (tx1 - tx0 + 1) * (ty1 - ty0 + 1);
             if (ntiles > (int)B.big_tiles) {
                 ntiles = 0;
@@ -606,9 +622,9 @@ __global__ __launch_bounds__(256) void k_front(BatchDev B, const JobDev *__restr
         }
         if (B.fixed) {
             const uint32_t rank = wave_add<true>(B.tile_count, key * SW_TILE_PAD, act);
-            if (act && rank < J.tile_cap)   // top bit: the raster must look at the marks
+            if (act && rank < J.tile_cap)
                 B.bins_fixed[J.bin_base + (size_t)(key - J.tile_base) * J.tile_cap + rank] =
-                    self_marked ? t : t | SW_BIN_CHECK;
+                    t | (self_marked ? 0u : SW_BIN_CHECK) | (large ? SW_BIN_LARGE : 0u);
             overflow |= act && rank >= J.tile_cap;
         } else {
             wave_add<false>(B.tile_count, key * SW_TILE_PAD, act);
@@ -799,16 +815,20 @@ __device__ __forceinline__ uint32_t slot_code(const Setup &S, uint32_t i0, uint3
         return SW_SLOT_NOPERM | (S.inverted ? 16u : 0u);
     return 3u * p0 + p1 + (S.inverted ? 16u : 0u);
 }
+__device__ __forceinline__ void store_slots(unsigned long long *slots, int n, int i, uint32_t tag, float u, float pl,
+                                            float pr)
+{
+    const uint64_t hi = (uint64_t)tag << 32;
+    __hip_atomic_store(&slots[i], hi | __float_as_uint(u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __hip_atomic_store(&slots[n + i], hi | __float_as_uint(pl), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __hip_atomic_store(&slots[2 * n + i], hi | __float_as_uint(pr), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
 __device__ __forceinline__ void put_slots(unsigned long long *slots, int n, int i, uint32_t seq, uint32_t code,
                                           bool lower, bool lr, float u, float pl, float pr)
 {
     if (seq > SW_SLOT_SEQ)
         return;
-    const uint64_t tag = (uint64_t)(seq | code << 25 | (lower ? 1u << 30 : 0u) | (lr ? 1u << 31 : 0u)) << 32;
-    __hip_atomic_store(&slots[i], tag | __float_as_uint(u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    __hip_atomic_store(&slots[n + i], tag | __float_as_uint(pl), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    __hip_atomic_store(&slots[2 * n + i], tag | __float_as_uint(pr), __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_WORKGROUP);
+    store_slots(slots, n, i, seq | code << 25 | (lower ? 1u << 30 : 0u) | (lr ? 1u << 31 : 0u), u, pl, pr);
 }
 
 // c ? a : b, field by field: a select of whole structs would take their
@@ -869,16 +889,12 @@ __device__ __forceinline__ void walk_rows(const Setup &S, int wy0, int wy1, RowF
     }
 }
 
-// check_mark: t came from a list that holds unmarked triangles too (the
-// marks are read beside the vertices, the triangle skipped when unmarked).
-__device__ void raster_depth(const JobDev &J, uint32_t t, TileRect tr, int wy0, int wy1,
-                             unsigned long long *keys, int TW, uint32_t &frags, uint32_t &nans,
-                             unsigned long long *slots = nullptr, int nslot = 0, bool check_mark = false)
+// Any triangle: near-clipped (two sub-triangles), non-finite, of any size.
+__device__ void raster_depth_any(const JobDev &J, uint32_t t, uint32_t i0, uint32_t i1, uint32_t i2, TileRect tr,
+                                 int wy0, int wy1, unsigned long long *keys, int TW, uint32_t &frags,
+                                 uint32_t &nans, unsigned long long *slots, int nslot)
 {
     SubTri st[2];
-    const uint32_t i0 = ro(J.tri)[3 * t], i1 = ro(J.tri)[3 * t + 1], i2 = ro(J.tri)[3 * t + 2];
-    if (check_mark && !((ro(J.yes)[i0] != 0) & (ro(J.yes)[i1] != 0) & (ro(J.yes)[i2] != 0)))
-        return;
     int ns = tri_subs_v<true>(J, i0, i1, i2, st);
 #pragma unroll
     for (int s = 0; s < 2; s++) {
@@ -919,6 +935,223 @@ __device__ void raster_depth(const JobDev &J, uint32_t t, TileRect tr, int wy0, 
                 }
             }
         });
+    }
+}
+
+// The job of a tile, its fields not known to have been read before: what a
+// later phase of the tile needs is then read when that phase begins, not
+// carried in scalar registers (and spilled to vector lanes) through the
+// phase before.
+__device__ __forceinline__ const JobDev &reread(const JobDev *__restrict__ jobs, int j)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(j));
+    j = __builtin_amdgcn_readfirstlane(j);
+#endif
+    return jobs[j];
+}
+
+// ------------------------------------------------- plain triangles
+// Plain triangles -- every vertex in front of the near plane, no coordinate
+// beyond 2^16, no depth beyond 2^20 and none more than 4 times another: all
+// but a few -- take a replay of their own.  They have one sub-triangle
+// without clip vertices, and every division on the way is in the range of
+// rcp_rn and div_rn (core.h): screen coordinates are multiples of 2^-26 (a
+// product near -m03 plus m03 >= 1/2), so heights and widths are zero or at
+// least that; over at most 2^17 adds the interpolators stay within 5 % of
+// the interval their ends span, so 1 / z stays positive and depths within a
+// factor of 6 of each other.  Only a span's width and first displacement,
+// differences of accumulated sums, are checked, per row.  Most entries are a
+// pixel or two, so the setup counts: reciprocals of the depths come with the
+// vertices, those of the heights serve slope and interpolator.  With the
+// shading's short forms the 999,698-triangle 1920x1080 field takes 31 M VALU
+// wave-instructions instead of 42 M and 88 us instead of 94 (what is left of
+// its raster is latency), four 1920x1080 views of 500,000 stacked triangles
+// 257 us instead of 316.
+struct PVert { float x, y, z, iz; };   // screen x and y, z, 1 / z
+struct PTri { PVert a, b, c; };
+__device__ __forceinline__ bool is_plain(const PTri &T)
+{
+    const float zmin = fminf(T.a.z, fminf(T.b.z, T.c.z)), zmax = fmaxf(T.a.z, fmaxf(T.b.z, T.c.z));
+    return (T.a.z >= SW_NEAR) & (T.b.z >= SW_NEAR) & (T.c.z >= SW_NEAR) & (zmax <= 0x1p20f) &
+           (zmax <= 4.0f * zmin) & (fabsf(T.a.x) <= 0x1p16f) & (fabsf(T.b.x) <= 0x1p16f) &
+           (fabsf(T.c.x) <= 0x1p16f) & (fabsf(T.a.y) <= 0x1p16f) & (fabsf(T.b.y) <= 0x1p16f) &
+           (fabsf(T.c.y) <= 0x1p16f);
+}
+
+// What the replay reads of a tile's job, held for a whole tile.
+struct TileView {
+    const uint32_t *tri;
+    const float4 *ndc;
+    const uint8_t *yes;
+    float m00, m03, m11, m13;
+    int vx, vy;
+    TileRect tr;
+};
+__device__ __forceinline__ PVert tile_vertex(const TileView &W, uint32_t i)
+{
+    const float4 f = ro4(W.ndc, i);
+    return {W.m00 * f.x + W.m03, W.m11 * f.y + W.m13, f.z, f.w};
+}
+
+// One side from vertex p to q, at the row m below p: Interp::init and
+// displace with 1 / z at hand and the reciprocal of the height shared by the
+// slope and the interpolator.
+struct PSide { float x, ratio, ta, ts, ba, bs, v0, v1; };
+__device__ __forceinline__ PSide plain_side(const PVert &p, const PVert &q, float m)
+{
+    const float d = q.y - p.y, r = rcp_rn(d);
+    PSide s;
+    s.ratio = div_rn(q.x - p.x, d, r);
+    s.ts = q.iz * r;
+    s.bs = (q.iz - p.iz) * r;
+    s.ta = s.ts * m;
+    s.ba = p.iz + s.bs * m;
+    s.x = p.x + s.ratio * m;
+    s.v0 = p.z;
+    s.v1 = q.z - p.z;
+    return s;
+}
+__device__ __forceinline__ void side_step(PSide &s)
+{
+    s.x += s.ratio;
+    s.ta += s.ts;
+    s.ba += s.bs;
+}
+__device__ __forceinline__ void side_steps(PSide &s, int n)
+{
+    int i = 0;
+    for (; i + 4 <= n; i += 4) {
+        side_step(s);
+        side_step(s);
+        side_step(s);
+        side_step(s);
+    }
+    for (; i < n; i++)
+        side_step(s);
+}
+
+// The fragments of plain triangle t (vertices i0, i1, i2) in rows [wy0, wy1)
+// of the tile.
+template <int TW, bool SLOTS>
+__device__ __forceinline__ void plain_depth(const TileView &W, const PTri &T, uint32_t t, uint32_t i0, uint32_t i1,
+                                            uint32_t i2, int wy0, int wy1, unsigned long long *keys,
+                                            unsigned long long *slots, int nslot, uint32_t &frags, uint32_t &nans)
+{
+    const PVert a = T.a, b = T.b, c = T.c;
+    // fill_triangle's facing (cross_z_sign, whose product is zero or at least
+    // 2^-52 here) and vertex order: the z-sort (renderer.cpp:262-279) only
+    // matters to the y-sort (:375-387) where two heights are equal
+    const bool front = (b.x - a.x) * (c.y - a.y) - (b.y - a.y) * (c.x - a.x) < 0.0f;
+    const bool ba = b.y < a.y, cb = c.y < b.y, ca = c.y < a.y;
+    bool a0 = !ba & !ca, b0 = ba & !cb, a2 = ba & ca, b2 = !ba & cb;   // a, b first; a, b last
+    if ((a.y == b.y) | (b.y == c.y) | (a.y == c.y)) {
+        uint32_t o0 = 0, o1 = 1, o2 = 2, x;
+        float z0 = a.z, z1 = b.z, z2 = c.z, y0 = a.y, y1 = b.y, y2 = c.y, f;
+        auto swap01 = [&] { x = o0; o0 = o1; o1 = x; f = z0; z0 = z1; z1 = f; f = y0; y0 = y1; y1 = f; };
+        auto swap12 = [&] { x = o1; o1 = o2; o2 = x; f = z1; z1 = z2; z2 = f; f = y1; y1 = y2; y2 = f; };
+        if (z1 > z0) swap01();
+        if (z2 > z1) swap12();
+        if (z1 > z0) swap01();
+        if (y1 < y0) swap01();
+        if (y2 < y1) swap12();
+        if (y1 < y0) swap01();
+        a0 = o0 == 0;
+        b0 = o0 == 1;
+        a2 = o2 == 0;
+        b2 = o2 == 1;
+    }
+    const bool a1 = !a0 & !a2, b1 = !b0 & !b2;
+    auto sel = [](bool m0, bool m1, float u, float v, float w) { return m0 ? u : m1 ? v : w; };
+    const PVert p0 = {sel(a0, b0, a.x, b.x, c.x), sel(a0, b0, a.y, b.y, c.y), sel(a0, b0, a.z, b.z, c.z),
+                      sel(a0, b0, a.iz, b.iz, c.iz)},
+                p1 = {sel(a1, b1, a.x, b.x, c.x), sel(a1, b1, a.y, b.y, c.y), sel(a1, b1, a.z, b.z, c.z),
+                      sel(a1, b1, a.iz, b.iz, c.iz)},
+                p2 = {sel(a2, b2, a.x, b.x, c.x), sel(a2, b2, a.y, b.y, c.y), sel(a2, b2, a.z, b.z, c.z),
+                      sel(a2, b2, a.iz, b.iz, c.iz)};
+    // fill_triangle_2: rows [ys, iy2) of the viewport, the short side
+    // changing at iy1 (walk_rows; the tile's rows lie inside the viewport's)
+    const int iy0 = (int)ceilf(p0.y), iy1 = (int)ceilf(p1.y), iy2 = (int)ceilf(p2.y);
+    const int ys = max(iy0, W.vy), ya = max(wy0, ys), yb = min(wy1, iy2);
+    if (ya >= yb)
+        return;
+    // tag of the payload slots (put_slots), without its row's bits
+    const uint32_t seq = 2u * t;
+    uint32_t tag0 = 0;
+    if (SLOTS) {
+        const uint32_t perm = 3u * (a0 ? 0u : b0 ? 1u : 2u) + (a1 ? 0u : b1 ? 1u : 2u);
+        tag0 = ((i0 == i1) | (i1 == i2) | (i0 == i2) ? SW_SLOT_NOPERM : perm) + (front ? 0u : 16u);
+        tag0 = seq | tag0 << 25;
+    }
+    const float m = (float)ys - p0.y;
+    PSide L = plain_side(p0, p2, m), S = plain_side(p0, p1, m);
+    const int yl = max(iy1, W.vy);
+    const PSide Sl = plain_side(p1, p2, (float)yl - p1.y);
+    bool lower = ya >= iy1, lr = L.ratio > S.ratio;
+    const bool lr_lo = L.ratio < Sl.ratio;
+    side_steps(L, ya - ys);
+    if (lower) {
+        S = Sl;
+        lr = lr_lo;
+    }
+    side_steps(S, ya - (lower ? yl : ys));
+    for (int y = ya; y < yb; y++) {
+        if (!lower & (y == iy1)) {
+            lower = true;
+            lr = lr_lo;
+            S = Sl;
+        }
+        // span_of: the row's columns, then its sides' progresses and depths
+        const float lx = lr ? S.x : L.x, rx = lr ? L.x : S.x;
+        const int x1 = max((int)ceilf(lx), W.vx);
+        const int xa = max(x1, W.tr.x0), xb = min((int)ceilf(rx), W.tr.x1);
+        if (xa < xb) {
+            const float uL = div_rn(L.ta, L.ba, rcp_rn(L.ba)), uS = div_rn(S.ta, S.ba, rcp_rn(S.ba));
+            const float zL = L.v0 + L.v1 * uL, zS = S.v0 + S.v1 * uS;
+            const float pl = lr ? uS : uL, pr = lr ? uL : uS, zl = lr ? zS : zL, zr = lr ? zL : zS;
+            const float dist = rx - lx, dx = (float)x1 - lx;
+            Interp q;
+            const bool fast = (dist >= 0x1p-20f) & ((dx == 0.0f) | (dx >= 0x1p-40f));
+            if (fast) {
+                const float as = rcp_rn(dist), iz2 = rcp_rn(zr);
+                q.ba = rcp_rn(zl);
+                q.v0 = zl;
+                q.v1 = zr - zl;
+                q.ts = iz2 * as;
+                q.bs = (iz2 - q.ba) * as;
+                q.ta = 0.0f;
+            } else {
+                q.init(dist, zl, zr);
+            }
+            q.displace(dx);
+            q.steps(xa - x1);
+            const int rowi = (y - W.tr.y0) * TW - W.tr.x0;
+            const uint32_t tag = tag0 | (lower ? 1u << 30 : 0u) | (lr ? 1u << 31 : 0u);
+            for (int x = xa; x < xb; x++, q.step()) {
+                const float u = fast ? div_rn(q.ta, q.ba, rcp_rn(q.ba)) : q.u();
+                const float z = q.value(u);
+                if (z < SW_NEAR)
+                    continue;
+                frags++;
+                if (!fast) {
+                    if (z != z) {
+                        nans++;
+                        continue;
+                    }
+                    if (__float_as_uint(z) >= SW_MAX_Z_BITS)
+                        continue;
+                }
+                const unsigned long long key = vis_key(z, seq);
+                if (SLOTS) {
+                    if (key < atomicMin(&keys[rowi + x], key) && seq <= SW_SLOT_SEQ)
+                        store_slots(slots, nslot, rowi + x, tag, u, pl, pr);
+                } else {
+                    atomicMin(&keys[rowi + x], key);
+                }
+            }
+        }
+        side_step(L);
+        side_step(S);
     }
 }
 
@@ -1119,6 +1352,7 @@ __device__ __forceinline__ void raster_tile(const BatchDev &B, const JobDev *__r
                                             unsigned long long *keys, uint32_t *s_cnt, unsigned long long *slots)
 {
     constexpr int NSLOT = TW * TH;
+    constexpr bool SLOTS = NSLOT <= 1024;   // as k_raster's
     const int jidx = find_job<JTILE>(B, jobs, g);
     const JobDev &J = jobs[jidx];
     const int lt = (int)(g - J.tile_base);
@@ -1135,12 +1369,19 @@ __device__ __forceinline__ void raster_tile(const BatchDev &B, const JobDev *__r
 
     uint32_t frags = 0, nans = 0, oob = 0;
     // Replay the tile's binned triangles, then the job's big triangles whose
-    // rectangle touches this tile.  With more than 256 of them, one lane per
-    // triangle.  With fewer, a triangle's rows in the tile are split into
-    // chunks of about 64 pixels (from its screen bounding box) and the chunks
-    // are dealt to the lanes, so a large triangle does not leave one lane
-    // looping over its pixels while the others idle.
-    __shared__ uint32_t s_tri[256], s_rows[256], s_first[256], s_wsum[4];
+    // rectangle touches this tile.  Up to 256 of them are cut into chunks of
+    // rows, of about an equal number of pixels (from the screen bounding
+    // boxes) and about as many as there are lanes, so that a few large
+    // triangles occupy every lane.  With more than 256, a lane takes a
+    // triangle of its own, all rows, if it is plain and not one that covers
+    // more than SW_LANE_PIXELS pixels of the tile, on which its lane would
+    // spend several times what the others do; those are listed and cut up
+    // after.  (Chunks of a fixed 64 pixels left a tile under 36 triangles 24 us
+    // in this phase with 20-40 lanes busy, and one lane per triangle a tile
+    // of 330 entries with one large among them 65 us.  The 640x480 cube's
+    // raster 45 -> 31 us, the 800x600 demo scene's 78 -> 47; chunks of at
+    // least 16 or 32 pixels: 34 and 40 us for the cube.)
+    __shared__ uint32_t s_tri[256], s_rows[256], s_first[256], s_wsum[4], s_n;
     // The tile's entries: placed by k_front in its job's fixed layout
     // (every triangle whose rectangle holds the tile; marks are checked
     // here), or, when a tile of the job passed its capacity, by k_bin_fill
@@ -1156,71 +1397,151 @@ __device__ __forceinline__ void raster_tile(const BatchDev &B, const JobDev *__r
         nb = B.tile_cursor[g * SW_TILE_PAD];
         bins = B.bins + B.tile_offset[g];
     }
-    const uint32_t nbig = B.ctr[SW_CTR_BIG0 + jidx];
+    const uint32_t entries = nb + B.ctr[SW_CTR_BIG0 + jidx];
     const int lane = __lane_id(), wave = threadIdx.x >> 6;
-    if (nb + nbig > 256) {
-        // enough triangles to fill the lanes: one lane per triangle, all rows
-        for (uint32_t e = threadIdx.x; e < nb + nbig; e += 256) {
+    TileView W;
+    W.tri = J.tri;
+    W.ndc = J.ndc;
+    W.yes = J.yes;
+    W.m00 = J.V.m00;
+    W.m03 = J.V.m03;
+    W.m11 = J.V.m11;
+    W.m13 = J.V.m13;
+    W.vx = J.V.vx;
+    W.vy = J.V.vy;
+    W.tr = tr;
+    // Triangle t's vertices, and whether it is drawn: `check`, its marks are
+    // still to be looked up.
+    auto load = [&](uint32_t t, bool check, uint32_t &i0, uint32_t &i1, uint32_t &i2, PTri &T) {
+        i0 = ro(W.tri)[3 * t];
+        i1 = ro(W.tri)[3 * t + 1];
+        i2 = ro(W.tri)[3 * t + 2];
+        T.a = tile_vertex(W, i0);
+        T.b = tile_vertex(W, i1);
+        T.c = tile_vertex(W, i2);
+        return !check || ((ro(W.yes)[i0] != 0) & (ro(W.yes)[i1] != 0) & (ro(W.yes)[i2] != 0));
+    };
+    // The tile rows a triangle covers and about how many of the tile's
+    // pixels: rows [ceil(ymin), ceil(ymax)) are exactly the rows
+    // fill_triangle_2 visits for an unclipped triangle; others (clipped,
+    // non-finite) keep all rows and columns of the tile.
+    auto rows_of = [&](const PTri &T, bool plain, int &ry0, int &ry1) {
+        int w = W.tr.x1 - W.tr.x0;
+        ry0 = W.tr.y0;
+        ry1 = W.tr.y1;
+        if (plain) {
+            ry0 = max(ry0, (int)ceilf(fminf(T.a.y, fminf(T.b.y, T.c.y))));
+            ry1 = min(ry1, (int)ceilf(fmaxf(T.a.y, fmaxf(T.b.y, T.c.y))));
+            const int xa = max(W.tr.x0, (int)floorf(fminf(T.a.x, fminf(T.b.x, T.c.x))));
+            const int xb = min(W.tr.x1, (int)ceilf(fmaxf(T.a.x, fmaxf(T.b.x, T.c.x))) + 1);
+            w = max(xb - xa, 1);
+        }
+        return max(ry1 - ry0, 0) * w;
+    };
+    // Entry e of the tile: its triangle, whether its marks are still to be
+    // looked up and whether it may cover many pixels (neither is ever set in
+    // the filled layout); false: a big triangle elsewhere.
+    auto entry = [&](uint32_t e, uint32_t &t, bool &check, bool &large) -> bool {
+        if (e < nb) {
+            const uint32_t k = ro(bins)[e], flags = fixed ? k & (SW_BIN_CHECK | SW_BIN_LARGE) : 0u;
+            t = k ^ flags;
+            check = (flags & SW_BIN_CHECK) != 0;
+            large = (flags & SW_BIN_LARGE) != 0;
+            return true;
+        }
+        const JobDev &B1 = reread(jobs, jidx);
+        t = ro(B1.big)[e - nb];
+        check = large = true;
+        const uint2 r = ro2(B1.rect, t);
+        return (tx >= (int)(r.x & 0xFFFF)) & (tx <= (int)(r.y & 0xFFFF)) & (ty >= (int)(r.x >> 16)) &
+               (ty <= (int)(r.y >> 16));
+    };
+    const bool many = entries > 256;
+    uint32_t listed = entries;
+    if (many) {
+        if (threadIdx.x == 0)
+            s_n = 0;
+        __syncthreads();
+        auto list = [&](uint32_t t) {
+            const uint32_t at = atomicAdd(&s_n, 1u);
+            if (at < 256u)
+                s_tri[at] = t;
+        };
+        // The loads of an entry are a chain of three (entry, vertex ids,
+        // vertices): the next entry's ids and the one after's entry are on
+        // their way while this one is replayed.
+        const uint32_t flags = fixed ? SW_BIN_CHECK | SW_BIN_LARGE : 0u;
+        if (threadIdx.x < nb) {
+            uint32_t e = threadIdx.x, k = ro(bins)[e], kn = ro(bins)[min(e + 256u, nb - 1u)];
+            uint32_t t = k & ~flags, i0 = ro(W.tri)[3 * t], i1 = ro(W.tri)[3 * t + 1], i2 = ro(W.tri)[3 * t + 2];
+            for (;; e += 256) {
+                PTri T;
+                T.a = tile_vertex(W, i0);
+                T.b = tile_vertex(W, i1);
+                T.c = tile_vertex(W, i2);
+                const uint32_t tn = kn & ~flags;
+                const uint32_t n0 = ro(W.tri)[3 * tn], n1 = ro(W.tri)[3 * tn + 1], n2 = ro(W.tri)[3 * tn + 2];
+                const uint32_t kn2 = ro(bins)[min(e + 512u, nb - 1u)];
+                const bool drawn = !(k & flags & SW_BIN_CHECK) ||
+                                   ((ro(W.yes)[i0] != 0) & (ro(W.yes)[i1] != 0) & (ro(W.yes)[i2] != 0));
+                if (drawn) {
+                    int ry0, ry1;
+                    if (!is_plain(T) ||
+                        ((k & flags & SW_BIN_LARGE) && rows_of(T, true, ry0, ry1) > SW_LANE_PIXELS))
+                        list(t);
+                    else
+                        plain_depth<TW, SLOTS>(W, T, t, i0, i1, i2, W.tr.y0, W.tr.y1, keys, slots, NSLOT, frags, nans);
+                }
+                if (e + 256 >= nb)
+                    break;
+                k = kn;
+                t = tn;
+                i0 = n0;
+                i1 = n1;
+                i2 = n2;
+                kn = kn2;
+            }
+        }
+        for (uint32_t e = nb + threadIdx.x; e < entries; e += 256) {
             uint32_t t;
-            bool check = false;
-            if (e < nb) {
-                t = ro(bins)[e];
-                check = (t & SW_BIN_CHECK) != 0;   // never set in the filled layout
-                t &= ~SW_BIN_CHECK;
-            } else {
-                t = ro(J.big)[e - nb];
-                const uint2 r = ro2(J.rect, t);
-                if (tx < (int)(r.x & 0xFFFF) || tx > (int)(r.y & 0xFFFF) || ty < (int)(r.x >> 16) ||
-                    ty > (int)(r.y >> 16) || !marked(J, t))
-                    continue;
-            }
-            raster_depth(J, t, tr, tr.y0, tr.y1, keys, TW, frags, nans, slots, NSLOT, check);
+            bool check, large;
+            if (entry(e, t, check, large) && marked(reread(jobs, jidx), t))
+                list(t);
         }
-    } else {
-    for (uint32_t base = 0; base < nb + nbig; base += 256) {
-        const uint32_t e = base + threadIdx.x;
-        uint32_t t = 0xFFFFFFFFu, nch = 0;
-        int ry0 = tr.y0, ry1 = tr.y1;
-        bool check = false;
-        if (e < nb + nbig) {
-            if (e < nb) {
-                t = ro(bins)[e];
-                check = (t & SW_BIN_CHECK) != 0;
-                t &= ~SW_BIN_CHECK;
-            } else {
-                t = ro(J.big)[e - nb];
-                const uint2 r = ro2(J.rect, t);
-                if (tx < (int)(r.x & 0xFFFF) || tx > (int)(r.y & 0xFFFF) || ty < (int)(r.x >> 16) ||
-                    ty > (int)(r.y >> 16) || !marked(J, t))
-                    t = 0xFFFFFFFFu;
+        __syncthreads();
+        listed = s_n;
+    }
+    // The listed triangles, 256 at a time.  More than 256 listed out of many
+    // are found again among the entries.
+    const bool again = many && listed > 256;
+    const uint32_t last = again ? entries : listed;
+    for (uint32_t base = 0; base < last; base += 256) {
+        uint32_t t = 0, area = 0;
+        int ry0 = tr.y0, ry1 = tr.y0;
+        if (base + threadIdx.x < last) {
+            uint32_t i0, i1, i2;
+            bool check = false, large = true, have = true;
+            PTri T;
+            if (many && !again)
+                t = s_tri[threadIdx.x];
+            else
+                have = entry(base + threadIdx.x, t, check, large);
+            if (have && load(t, check, i0, i1, i2, T)) {   // unmarked: no chunks
+                const bool plain = is_plain(T);
+                area = (uint32_t)rows_of(T, plain, ry0, ry1);
+                if (again && base + threadIdx.x < nb && plain && !(large && area > SW_LANE_PIXELS))
+                    area = 0;   // done above
             }
         }
-        if (t != 0xFFFFFFFFu) {
-            // rows [ceil(ymin), ceil(ymax)) are exactly the rows fill_triangle_2 visits for an
-            // unclipped triangle; clipped or non-finite ones keep all rows of the tile
-            const uint32_t i0 = ro(J.tri)[3 * t], i1 = ro(J.tri)[3 * t + 1], i2 = ro(J.tri)[3 * t + 2];
-            if (check && !((ro(J.yes)[i0] != 0) & (ro(J.yes)[i1] != 0) & (ro(J.yes)[i2] != 0)))
-                t = 0xFFFFFFFFu;   // unmarked: no chunks
-        }
-        if (t != 0xFFFFFFFFu) {
-            const uint32_t i0 = ro(J.tri)[3 * t], i1 = ro(J.tri)[3 * t + 1], i2 = ro(J.tri)[3 * t + 2];
-            const f3 a = frustum_to_screen(J.V, ld3(J.ndc, i0)), b = frustum_to_screen(J.V, ld3(J.ndc, i1)),
-                     c = frustum_to_screen(J.V, ld3(J.ndc, i2));
-            const float big = 1073741824.0f;
-            int w = tr.x1 - tr.x0;
-            if (fabsf(a.y) < big && fabsf(b.y) < big && fabsf(c.y) < big && fabsf(a.x) < big &&
-                fabsf(b.x) < big && fabsf(c.x) < big && fminf(a.z, fminf(b.z, c.z)) >= SW_NEAR) {
-                ry0 = max(tr.y0, cvtt(ceilf(fminf(a.y, fminf(b.y, c.y)))));
-                ry1 = min(tr.y1, cvtt(ceilf(fmaxf(a.y, fmaxf(b.y, c.y)))));
-                const int xa = max(tr.x0, (int)floorf(fminf(a.x, fminf(b.x, c.x))));
-                const int xb = min(tr.x1, (int)ceilf(fmaxf(a.x, fmaxf(b.x, c.x))) + 1);
-                w = max(xb - xa, 1);
-            }
-            const int rows = ry1 - ry0;
-            nch = rows > 0 ? (uint32_t)min(max(rows * w / 64, 1), rows) : 0u;
-        }
-        if (nch == 0)
-            ry0 = ry1 = tr.y0;
+        // pixels of a chunk: an equal share of the list's for every lane
+        const uint32_t sum = wave_sum(area);
+        if (lane == 0)
+            s_wsum[wave] = sum;
+        __syncthreads();
+        const uint32_t per = max((s_wsum[0] + s_wsum[1] + s_wsum[2] + s_wsum[3]) / 256u, (uint32_t)SW_CHUNK_PIXELS);
+        const uint32_t rows = (uint32_t)(ry1 - ry0);
+        const uint32_t nch = area ? min(max(area / per, 1u), rows) : 0u;
+        __syncthreads();   // s_wsum read, s_tri too
         // exclusive prefix of the chunk counts over the block
         const uint32_t incl = wave_incl_scan(nch);
         if (lane == 63)
@@ -1247,15 +1568,23 @@ __device__ __forceinline__ void raster_tile(const BatchDev &B, const JobDev *__r
             // s_first is non-decreasing and i < total, so entry lo has a chunk holding i
             // (an entry without chunks shares its s_first with the next entry)
             const uint32_t pk = s_rows[lo], n = pk >> 16, ch = i - s_first[lo];
-            const int r0 = tr.y0 + (int)(pk & 0xFF), rows = (int)((pk >> 8) & 0xFF) - (int)(pk & 0xFF);
-            const int ya = r0 + (int)((uint32_t)rows * ch / n), yb = r0 + (int)((uint32_t)rows * (ch + 1) / n);
-            raster_depth(J, s_tri[lo], tr, ya, yb, keys, TW, frags, nans, slots, NSLOT);
+            const int r0 = tr.y0 + (int)(pk & 0xFF), nr = (int)((pk >> 8) & 0xFF) - (int)(pk & 0xFF);
+            const int wy0 = r0 + (int)((uint32_t)nr * ch / n), wy1 = r0 + (int)((uint32_t)nr * (ch + 1) / n);
+            const uint32_t tt = s_tri[lo];
+            uint32_t i0, i1, i2;
+            PTri T;
+            load(tt, false, i0, i1, i2, T);
+            if (is_plain(T))
+                plain_depth<TW, SLOTS>(W, T, tt, i0, i1, i2, wy0, wy1, keys, slots, NSLOT, frags, nans);
+            else
+                raster_depth_any(reread(jobs, jidx), tt, i0, i1, i2, tr, wy0, wy1, keys, TW, frags, nans,
+                                 SLOTS ? slots : nullptr, NSLOT);
         }
-        __syncthreads();   // the LDS tables are rewritten by the next 256 entries
-    }
+        __syncthreads();   // the LDS tables are rewritten by the next 256
     }
     __syncthreads();
 
+    const JobDev &K = reread(jobs, jidx);
     const float maxz = __uint_as_float(SW_MAX_Z_BITS);
     for (int i = threadIdx.x; i < TW * TH; i += 256) {
         const int x = tr.x0 + (i % TW), y = tr.y0 + (i / TW);
@@ -1269,37 +1598,38 @@ __device__ __forceinline__ void raster_tile(const BatchDev &B, const JobDev *__r
             seq = (uint32_t)k;
             z = __uint_as_float((uint32_t)(k >> 32));
             bool done = false;
-            if (slots) {
+            if (SLOTS) {
                 const unsigned long long a = slots[i], b = slots[NSLOT + i], c = slots[2 * NSLOT + i];
                 const uint32_t tag = (uint32_t)(a >> 32);
                 if (tag == (uint32_t)(b >> 32) && tag == (uint32_t)(c >> 32) && (tag & SW_SLOT_SEQ) == seq) {
-                    color = shade_recorded<GENERIC>(J, seq, tag, __uint_as_float((uint32_t)a),
+                    color = shade_recorded<GENERIC>(K, seq, tag, __uint_as_float((uint32_t)a),
                                                     __uint_as_float((uint32_t)b), __uint_as_float((uint32_t)c), oob);
                     done = true;
                 }
             }
             if (!done)
-                color = shade_pixel<GENERIC>(J, seq, x, y, oob);
+                color = shade_pixel<GENERIC>(K, seq, x, y, oob);
         }
-        J.out_color[(int64_t)(y - J.out_oy) * J.out_pitch + (x - J.out_ox)] = color;
-        const int64_t zo = (int64_t)(y - J.V.vy) * J.V.vw + (x - J.V.vx);
-        J.zbuf[zo] = z;
-        if (J.tid)
-            J.tid[zo] = seq;
+        K.out_color[(int64_t)(y - K.out_oy) * K.out_pitch + (x - K.out_ox)] = color;
+        const int64_t zo = (int64_t)(y - K.V.vy) * K.V.vw + (x - K.V.vx);
+        K.zbuf[zo] = z;
+        if (K.tid)
+            K.tid[zo] = seq;
     }
     // The depth-of-field pass reads this code instead of z.  A loop of its
     // own keeps its registers out of the shading loop's peak.
-    if (J.dofc) {
-        const FDiv dof_by(J.fdepth - 1.0f);
-        const bool dof_fast = J.fdepth - 1.0f >= 1.0f && J.fdepth - 1.0f <= 0x1p20f;
+    const JobDev &D = reread(jobs, jidx);
+    if (D.dofc) {
+        const FDiv dof_by(D.fdepth - 1.0f);
+        const bool dof_fast = D.fdepth - 1.0f >= 1.0f && D.fdepth - 1.0f <= 0x1p20f;
         for (int i = threadIdx.x; i < TW * TH; i += 256) {
             const int x = tr.x0 + (i % TW), y = tr.y0 + (i / TW);
             if (x >= tr.x1 || y >= tr.y1)
                 continue;
             const float z = __uint_as_float((uint32_t)(keys[i] >> 32));   // max_z where empty
-            const float bf = blur_factor(z, J.fdist, J.fdepth, (float)J.rmax, dof_by, dof_fast);
-            const int radius = min(max(cvtt(bf), 0), J.rmax);   // bf is in [0, rmax] for finite inputs
-            J.dofc[(int64_t)(y - J.V.vy) * J.V.vw + (x - J.V.vx)] = (uint8_t)((bf != 0.0f ? 1 : 0) | (radius << 1));
+            const float bf = blur_factor(z, D.fdist, D.fdepth, (float)D.rmax, dof_by, dof_fast);
+            const int radius = min(max(cvtt(bf), 0), D.rmax);   // bf is in [0, rmax] for finite inputs
+            D.dofc[(int64_t)(y - D.V.vy) * D.V.vw + (x - D.V.vx)] = (uint8_t)((bf != 0.0f ? 1 : 0) | (radius << 1));
         }
     }
     if (B.stats) {
@@ -1363,7 +1693,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         const uint32_t g = s_tile;
         if (g == 0xFFFFFFFFu)
             break;
-        raster_tile<TW, TH, GENERIC>(B, jobs, g, keys, s_cnt, SLOTS ? slots : nullptr);
+        raster_tile<TW, TH, GENERIC>(B, jobs, g, keys, s_cnt, slots);
         __syncthreads();   // tile done with keys and s_tile before the next claim
     }
     __syncthreads();
@@ -1378,14 +1708,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 }
 
 // ------------------------------------------------------- k_raster_layers
-__device__ __forceinline__ uint32_t wave_sum(uint32_t v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
-        v += __shfl_xor(v, o);
-    return v;
-}
-
 // One pixel's base and layers (renderer.cpp:486-550)
 struct LayerPixel {
     float bz, lz[SW_MAX_LAYERS];

@@ -38,7 +38,12 @@ SW_HD float pow32(float s)
 
 struct Light4 { float x, y, z, I; };
 
-// pixel_shader_lights_phong::shade (pixel_shaders.cpp:159-205)
+// pixel_shader_lights_phong::shade (pixel_shaders.cpp:159-205).  The two
+// quotients over a light's squared distance d2 share its reciprocal where
+// div_rn holds: d2 and the intensity within [2^-40, 2^40], and the second
+// numerator, which may be tiny, scaled by 2^64 (exact) and the quotient
+// scaled back: exact again unless it is below the normal range, a band of
+// s^32 that takes the plain division.
 SW_D int32_t phong(f3 center, f3 normal, f3 cam, float ambient, f3 sun, float sun_I,
                    const Light4 *lights, int n_lights)
 {
@@ -52,11 +57,18 @@ SW_D int32_t phong(f3 center, f3 normal, f3 cam, float ambient, f3 sun, float su
     for (int i = 0; i < n_lights; i++) {
         const Light4 l = ro(lights)[i];
         f3 L = center - f3{l.x, l.y, l.z};
-        float d2 = L.x * L.x + L.y * L.y + L.z * L.z;
-        float diffuse = l.I / d2;
+        const float d2 = L.x * L.x + L.y * L.y + L.z * L.z;
+        const bool fast = d2 >= 0x1p-40f && d2 <= 0x1p40f && fabsf(l.I) >= 0x1p-40f && fabsf(l.I) <= 0x1p40f;
+        float r2 = 0.0f, diffuse;
+        if (fast) {
+            r2 = rcp_rn(d2);
+            diffuse = div_rn(l.I, d2, r2);
+        } else {
+            diffuse = l.I / d2;
+        }
         if (diffuse < SW_DIFFUSE_CUT)
             continue;
-        L = normalize(L);
+        L = normalize_s(L, d2);
         float a = -dot(normal, L);
         if (a < 0.0f)
             continue;
@@ -66,7 +78,12 @@ SW_D int32_t phong(f3 center, f3 normal, f3 cam, float ambient, f3 sun, float su
         if (s > 0) {
             s = pow32(s);
             s = s * 32.0f / 2.0f;
-            acc += diffuse + s / d2;
+            const float q = div_rn(s * 0x1p64f, d2, r2);
+            if (fast && s <= 0x1p10f && (q >= 0x1p-62f || s == 0.0f))
+                s = q * 0x1p-64f;
+            else
+                s = s / d2;
+            acc += diffuse + s;
         } else {
             acc += diffuse;
         }
@@ -77,12 +94,17 @@ SW_D int32_t phong(f3 center, f3 normal, f3 cam, float ambient, f3 sun, float su
 // pixel_shader_texture_bilinear::shade (pixel_shaders.cpp:348-384).  The
 // reference reads outside the bitmap for coordinates that wrap to a negative
 // index (UB); here such a tap is clamped and counted.
-// x % m (C remainder); a mask when m is a power of two and x >= 0.
-SW_D int rem(int x, int m)
+// (x + m) % m with the reference's wrapping add and C remainder: x itself
+// when it lies in [0, m) already (no division: the common case of
+// coordinates inside the texture), a mask when m is a power of two.
+SW_D int wrap_mod(int x, int m)
 {
-    if (x >= 0 && (m & (m - 1)) == 0)
-        return x & (m - 1);
-    return x % m;
+    if ((uint32_t)x < (uint32_t)m)
+        return x;
+    const int s = wrap_add(x, m);
+    if (s >= 0 && (m & (m - 1)) == 0)
+        return s & (m - 1);
+    return s % m;
 }
 
 // A texture as the shaders read it: w x h texels at p, or, with p null, the
@@ -116,28 +138,43 @@ SW_D BilTaps bilinear_taps(const TexView &X, f2 t, uint32_t &oob)
     float v2 = v + 0.5f;
     u = floorf(u2);
     v = floorf(v2);
-    int v1m = rem(wrap_add(cvtt(v1), th), th);
+    int v1m = wrap_mod(cvtt(v1), th);
     int v2m = v1m + 1;
     if (v2m == th)
         v2m = 0;
-    v1m *= tw;
-    v2m *= tw;
-    int u1m = rem(wrap_add(cvtt(u1), tw), tw);
+    const int u1m = wrap_mod(cvtt(u1), tw);
     int u2m = u1m + 1;
     if (u2m == tw)
         u2m = 0;
-    const int64_t lim = (int64_t)tw * th;
-    int64_t idx[4] = {(int64_t)v1m + u1m, (int64_t)v2m + u1m, (int64_t)v1m + u2m,
-                      (int64_t)v2m + u2m};
     BilTaps T;
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        int64_t i = idx[k];
-        if (i < 0 || i >= lim) {
-            oob++;
-            i = i < 0 ? 0 : lim - 1;
+    if ((v1m | u1m) >= 0 && (tw | th) < 32768) {
+        // both taps of either axis inside the bitmap, and products of 30
+        // bits at most: 24-bit multiplies and 32-bit indices
+        const uint32_t r1 = __umul24((uint32_t)v1m, (uint32_t)tw), r2 = __umul24((uint32_t)v2m, (uint32_t)tw);
+        const uint32_t i0 = r1 + (uint32_t)u1m, i1 = r2 + (uint32_t)u1m, i2 = r1 + (uint32_t)u2m,
+                       i3 = r2 + (uint32_t)u2m;
+        T.p[0] = T.p[1] = T.p[2] = T.p[3] = X.one;
+        if (X.p) {
+            T.p[0] = ro(X.p)[i0];
+            T.p[1] = ro(X.p)[i1];
+            T.p[2] = ro(X.p)[i2];
+            T.p[3] = ro(X.p)[i3];
         }
-        T.p[k] = texel(X, i);
+    } else {
+        const int64_t lim = (int64_t)tw * th;
+        v1m *= tw;
+        v2m *= tw;
+        int64_t idx[4] = {(int64_t)v1m + u1m, (int64_t)v2m + u1m, (int64_t)v1m + u2m,
+                          (int64_t)v2m + u2m};
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            int64_t i = idx[k];
+            if (i < 0 || i >= lim) {
+                oob++;
+                i = i < 0 ? 0 : lim - 1;
+            }
+            T.p[k] = texel(X, i);
+        }
     }
     T.w[0] = (u - u1) * (v - v1);
     T.w[1] = (u - u1) * (v2 - v);
@@ -153,8 +190,13 @@ SW_D uint32_t bilinear_channel(const BilTaps &T, int c)
     float b = (float)((T.p[1] >> (8 * c)) & 0xFF) * T.w[1];
     float d = (float)((T.p[2] >> (8 * c)) & 0xFF) * T.w[2];
     float e = (float)((T.p[3] >> (8 * c)) & 0xFF) * T.w[3];
-    float s = ((a + b) + d) + e;
-    return (uint32_t)to_u8(roundf(s));
+    const float s = ((a + b) + d) + e;
+    // roundf (halves away from zero) and the conversion to a byte through a
+    // 32-bit int: s is never negative (the weights are not), so it is the
+    // integer part, plus one when the fraction, exact, reaches a half; NaN
+    // gives 0 as the conversion does
+    const float f = floorf(s);
+    return ((uint32_t)(int32_t)f + (s - f >= 0.5f ? 1u : 0u)) & 0xFFu;
 }
 
 SW_D uint32_t bilinear(const TexView &X, f2 t, uint32_t &oob)
@@ -204,21 +246,22 @@ SW_D uint32_t combine(uint32_t color, int32_t light_i)
     // scaled by 2^-16, which the float operations below reproduce exactly.
     float light = (float)light_i * 0x1p-16f;
     uint32_t out = color & 0xFF000000u;
+    // Conversions to int need no range check here: |c * light| < 2^24 (light
+    // is an int32 over 2^16), and the quotients below lie in [0, 255].
     if (light < 1) {
 #pragma unroll
         for (int k = 0; k < 3; k++) {
             uint32_t c = (color >> (8 * k)) & 0xFF;
-            out |= (uint32_t)to_u8((float)c * light) << (8 * k);
+            out |= ((uint32_t)(int32_t)((float)c * light) & 0xFFu) << (8 * k);
         }
     } else {
-        light = sqrtf(light);
-        light = sqrtf(light);
-        const FDiv by_light(light);   // 1 <= light <= 32768^(1/4); 0 <= 255 - c <= 255
+        light = sqrt_rn(light);   // 1 <= light <= 32768
+        light = sqrt_rn(light);
+        const FDiv by_light(light);
 #pragma unroll
         for (int k = 0; k < 3; k++) {
             uint32_t c = (color >> (8 * k)) & 0xFF;
-            uint8_t r = (uint8_t)(255 - to_u8(by_light((float)(255 - (int)c))));
-            out |= (uint32_t)r << (8 * k);
+            out |= (255u - (uint32_t)(int32_t)by_light((float)(255 - (int)c))) << (8 * k);
         }
     }
     return out;

@@ -1,0 +1,101 @@
+"""The raster's replay of plain triangles and its ways into a tile: tiles of
+at most and of more than 256 entries, with few, many and more than 256
+triangles that are listed and cut into chunks of rows (large ones, and ones
+that are not plain: near-clipped, of depths far apart, with coordinates far
+outside), equal heights and depths, and texture coordinates that are not
+finite.  Depth bits and winners equal the oracle's.  The short exact division
+and square root it rests on are compared with the IEEE ones on the device."""
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+import oracle
+from swegl_amd.device import Context
+
+from _helpers import compare, gpu_render
+from test_oracle_scene import flat_scene, view
+
+pytestmark = pytest.mark.gpu
+CPP = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp")
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = Context(0)
+    yield c
+    c.close()
+
+
+def triangles(rng, n, size, centre=(0.0, 0.0), spread=0.25, z=(-1.0, 0.5)):
+    """n random triangles of about `size` around points near `centre`."""
+    c = np.concatenate([rng.uniform(-spread, spread, (n, 1, 2)) + centre, rng.uniform(*z, (n, 1, 1))], -1)
+    return c + rng.uniform(-size, size, (n, 3, 3)) * [1, 1, 0.3]
+
+
+def crowd(kind, rng):
+    tiny = triangles(rng, 700, 0.03)
+    if kind == "tiny":
+        return tiny
+    if kind == "few":
+        return triangles(rng, 90, 0.4)
+    if kind == "mixed":
+        return np.concatenate([tiny, triangles(rng, 6, 0.9)])
+    if kind == "large":
+        return triangles(rng, 600, 0.7)
+    if kind == "near":
+        cut = triangles(rng, 350, 0.3)
+        cut[:, 0, 2] = rng.uniform(2.6, 3.4, 350)   # the camera is at z = 3
+        return np.concatenate([tiny, cut])
+    if kind == "deep":
+        far = triangles(rng, 350, 0.3)
+        far[:, 1, 2] = rng.uniform(-60.0, -8.0, 350)
+        far[:, 2, 2] = rng.uniform(2.2, 2.4, 350)
+        return np.concatenate([tiny, far])
+    if kind == "wide":
+        wide = triangles(rng, 300, 0.3)
+        wide[:, 2, 0] += rng.choice([-1.0, 1.0], 300) * 10.0 ** rng.uniform(1, 6, 300)
+        return np.concatenate([tiny, wide])
+    assert kind == "ties"
+    grid = rng.integers(-4, 5, (800, 3, 3)) * [0.125, 0.125, 0.25]   # many equal heights and depths
+    return grid
+
+
+@pytest.mark.parametrize("entry", ["swegl_render", "swegl_render_noalloc"])
+@pytest.mark.parametrize("kind", ["tiny", "few", "mixed", "large", "near", "deep", "wide", "ties"])
+def test_crowded_tiles(ctx, kind, entry):
+    rng = np.random.default_rng(sum(map(ord, kind)))
+    s = flat_scene(crowd(kind, rng).tolist(), double_sided=True)
+    vps = [view(83, 61)]
+    want = oracle.render(s, vps)
+    for limit in (16, 2):   # 2: the larger ones go to the viewport's big list
+        ctx.set_bin_limit(limit)
+        try:
+            got = gpu_render(ctx, s, vps, entry=entry)
+        finally:
+            ctx.set_bin_limit(16)
+        compare(got[0], want[0])
+        assert got[0].stats["fragments"] == want[0].stats["fragments"]
+
+
+def test_texture_coordinates_not_finite(ctx):
+    rng = np.random.default_rng(5)
+    s = flat_scene(triangles(rng, 40, 0.4).tolist(), double_sided=True)
+    p = s.nodes[0].primitives[0]
+    uv = rng.uniform(-3, 3, p.tex_coords.shape).astype(np.float32)
+    uv[::7] = [np.nan, 0.5]
+    uv[3::11] = [0.25, np.inf]
+    uv[5::13] = [-3e8, 2e7]
+    p.tex_coords[...] = uv
+    vps = [view(70, 50)]
+    want = oracle.render(s, vps)
+    compare(gpu_render(ctx, s, vps)[0], want[0])
+
+
+def test_short_forms_equal_ieee():
+    exe = os.path.join(CPP, "arith_check")
+    if not os.path.exists(exe):
+        subprocess.run(["make", "-C", CPP, "arith_check"], check=True, capture_output=True)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr
