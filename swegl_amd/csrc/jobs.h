@@ -116,7 +116,9 @@ struct WorldArgs {
 // Tile counters: tile g's bin count at tile_count[g * SW_TILE_PAD] and its
 // fill rank (entries placed so far) one word later, a 128-byte line per tile, so the binning
 // atomics of different tiles spread over all memory channels instead of
-// queueing on the few that a dense array maps to.
+// queueing on the few that a dense array maps to.  Words 4 to 7 of line i hold
+// slots 4i to 4i + 3 of the raster's claim order (item_slot), written by
+// k_bin_fill's first blocks.
 #define SW_TILE_PAD 32
 
 struct BatchDev {
@@ -125,7 +127,6 @@ struct BatchDev {
     uint32_t n_tiles;         // total tiles over all jobs
     uint32_t *tile_count;     // [n_tiles * SW_TILE_PAD], see SW_TILE_PAD
     uint32_t *tile_offset;    // [n_tiles + 1]
-    uint32_t *tile_order;     // [n_tiles]: tiles by descending bin count (k_bin_fill's last block), the raster's claim order
     uint32_t *tile_cursor;    // tile_count + 1: the fill ranks
     uint32_t *bins;           // [capacity]: the counted, scanned and filled layout
     uint32_t *bins_fixed;     // the fixed layout's entries (JobDev::bin_base, tile_cap)
@@ -139,7 +140,18 @@ struct BatchDev {
     // SW_CTR_OVERFLOW) is filled by k_bin_fill into the counted layout,
     // after the offsets scan; 0: the counted layout for every job
     uint32_t fixed;
+    uint32_t order;           // 1: k_bin_fill writes the claim order (0: layered waves, which have none)
+    uint32_t split;           // a tile of more entries is SW_BANDS items; 0xFFFFFFFF: none is
+    uint32_t n_static;        // raster workgroups that begin with an item of their own (launch_raster)
 };
+
+// An item of the claim order: a tile (its low SW_ITEM_BAND bits), whole, or
+// its rows' band b of SW_BANDS with b + 1 in the bits above.  Tiles are split
+// where they are at least 32 rows high and there are fewer than 2^28 of them.
+#define SW_BANDS 4
+#define SW_ITEM_BAND 28
+// Empty tiles taken per claim
+#define SW_EMPTY_CLAIM 8u
 
 // Counter block: [0, 1024) statistics as 64 slots x 8 u64 (slot = block
 // index mod 64, so no address takes one atomic per block; the host sums the
@@ -157,6 +169,10 @@ struct BatchDev {
 // its own 128-byte line (same-address atomics serialise where they execute)
 #define SW_TICKET_GROUPS 32
 #define SW_CTR_OVERFLOW (SW_CTR_TOTAL + 32)   // nonzero: a tile passed tile_cap
+// Each raster queue's number of items, then of empty tiles after them; the
+// claims of those (a line of its own for each queue)
+#define SW_CTR_ITEMS (SW_CTR_TOTAL + 34)
+#define SW_CTR_EMPTYQ (SW_CTR_TOTAL + 64)
 // A fixed-layout bin entry with this bit set names a triangle that failed its
 // own visibility test: it is drawn only if other triangles marked all three
 // of its vertices, which the raster looks up
@@ -164,7 +180,7 @@ struct BatchDev {
 // and one with this bit set a triangle whose bounding box holds more than
 // SW_LANE_PIXELS pixels (a job of the fixed layout holds < 2^30 triangles)
 #define SW_BIN_LARGE 0x40000000u
-#define SW_CTR_TICKETS (SW_CTR_TOTAL + 64)
+#define SW_CTR_TICKETS (SW_CTR_EMPTYQ + 32 * SW_RASTER_QUEUES)
 #define SW_CTR_BIG0 (SW_CTR_TICKETS + 32 * (SW_TICKET_GROUPS + 1))
 // statistic indices within a slot
 #define SW_ST_FRAGMENTS 0

@@ -12,6 +12,8 @@
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "jobs.h"
 #include "launch.h"
 
@@ -435,16 +437,18 @@ __device__ __forceinline__ uint32_t count_bucket(uint32_t c)
     return 4u * (e - 1u) + ((c >> (e - 2u)) & 3u);   // <= 123
 }
 
-// SCAN_PER consecutive tile counts from tile i0 on (zero past n), read with
+// The counts of tiles i * step + first for SCAN_PER consecutive i from i0 on
+// (zero past n), read with
 // device-scope atomic loads (the counts were added at the memory side in
 // this same kernel: an XCD's L2 may hold older lines), all issued before
 // the first is used.
-__device__ __forceinline__ void load_counts(const BatchDev &B, uint32_t i0, uint32_t n, uint32_t (&v)[SCAN_PER])
+__device__ __forceinline__ void load_counts(const BatchDev &B, uint32_t i0, uint32_t n, uint32_t (&v)[SCAN_PER],
+                                            uint32_t step = 1, uint32_t first = 0)
 {
 #pragma unroll
     for (int k = 0; k < SCAN_PER; k++)
-        v[k] = i0 + k < n ? __hip_atomic_load(&B.tile_count[(i0 + k) * SW_TILE_PAD], __ATOMIC_RELAXED,
-                                              __HIP_MEMORY_SCOPE_AGENT)
+        v[k] = i0 + k < n ? __hip_atomic_load(&B.tile_count[(size_t)((i0 + k) * step + first) * SW_TILE_PAD],
+                                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
                           : 0u;
 }
 
@@ -500,49 +504,87 @@ __device__ void scan_offsets(const BatchDev &B)
     }
 }
 
-// The raster's claim order, by one block of NT threads: the tiles sorted by
-// a log bucket of their bin counts, the largest bucket first (order within
-// a bucket is arbitrary: the raster's result does not depend on the claim
-// order).
-template <int NT>
-__device__ void order_tiles(const BatchDev &B)
+// The raster's claim order, by SW_RASTER_QUEUES blocks of NT threads, block q
+// for the tiles that are q mod SW_RASTER_QUEUES: one queue each, and an
+// eighth of the counter lines to read (a block reads a line every 2.5 ns or
+// so: one block for 8,160 tiles took 42 us).  A queue's items are sorted by
+// a log bucket of their bin counts, the largest bucket first (order within a
+// bucket is arbitrary: the raster's result does not depend on the claim
+// order), then come its empty tiles.
+// A tile of more than B.split entries is SW_BANDS items, a band of its rows
+// each, so that the replay of a crowded tile -- a chain of 10 to 40 entries
+// a lane -- is spread over several workgroups; an entry outside a band's
+// rows costs little there.  Tiles without entries, where no job has big
+// triangles either, are kept apart: the raster fills them without a claim
+// each.
+// Place j of queue q is slot 8 j + q; four slots lie in each tile's counter
+// line, which has room (a tile is at most SW_BANDS items).
+static_assert(SW_BANDS == 4 && SW_TILE_PAD >= 8, "four slots a counter line");
+__device__ __forceinline__ uint32_t *item_slot(const BatchDev &B, uint32_t p)
 {
-    __shared__ uint32_t s_hist[SW_ORDER_BUCKETS];
-    const uint32_t n = B.n_tiles;
+    return B.tile_count + (size_t)(p >> 2) * SW_TILE_PAD + 4 + (p & 3);
+}
+template <int NT>
+__device__ void order_tiles(const BatchDev &B, uint32_t queue)
+{
+    constexpr uint32_t Q = SW_RASTER_QUEUES;
+    __shared__ uint32_t s_hist[SW_ORDER_BUCKETS], s_big;
+    const uint32_t n = B.n_tiles > queue ? (B.n_tiles - 1u - queue) / Q + 1u : 0u;
     const int lane = __lane_id(), wave = threadIdx.x >> 6;
+    if (threadIdx.x == 0)
+        s_big = 0;
     for (int b = threadIdx.x; b < SW_ORDER_BUCKETS; b += NT)
         s_hist[b] = 0;
     __syncthreads();
+    uint32_t big = 0;
+    for (uint32_t j = threadIdx.x; j < B.n_jobs; j += NT)
+        big |= B.ctr[SW_CTR_BIG0 + j];
+    if (big)
+        s_big = 1;
+    auto bands = [&](uint32_t c) { return c > B.split ? (uint32_t)SW_BANDS : 1u; };
     uint32_t v[SCAN_PER];
     for (uint32_t base = 0; base < n; base += (uint32_t)NT * SCAN_PER) {
         const uint32_t i0 = base + threadIdx.x * SCAN_PER;
-        load_counts(B, i0, n, v);
+        load_counts(B, i0, n, v, Q, queue);
 #pragma unroll
         for (int k = 0; k < SCAN_PER; k++)
             if (i0 + k < n)
-                atomicAdd(&s_hist[count_bucket(v[k])], 1u);
+                atomicAdd(&s_hist[count_bucket(v[k] / bands(v[k]))], bands(v[k]));
     }
     __syncthreads();
     // first place of each bucket, the largest bucket first: wave 0 scans the
-    // buckets in descending order, two per lane
+    // buckets in descending order, two per lane; the last bucket holds the
+    // empty tiles
     if (wave == 0) {
         const int b0 = SW_ORDER_BUCKETS - 1 - 2 * lane, b1 = b0 - 1;
         const uint32_t h0 = s_hist[b0], h1 = s_hist[b1];
         const uint32_t incl = wave_incl_scan(h0 + h1);
         s_hist[b0] = incl - h0 - h1;
         s_hist[b1] = incl - h1;
+        if (lane == 63) {
+            const uint32_t items = s_big ? incl : incl - h1;
+            B.ctr[SW_CTR_ITEMS + 2 * queue] = items;
+            B.ctr[SW_CTR_ITEMS + 2 * queue + 1] = incl - items;
+        }
     }
     __syncthreads();
-    // every tile takes the next place of its bucket; with one pass the
+    // every tile takes the next places of its bucket; with one pass the
     // counts are still in registers
     for (uint32_t base = 0; base < n; base += (uint32_t)NT * SCAN_PER) {
         const uint32_t i0 = base + threadIdx.x * SCAN_PER;
         if (n > (uint32_t)NT * SCAN_PER)
-            load_counts(B, i0, n, v);
+            load_counts(B, i0, n, v, Q, queue);
 #pragma unroll
         for (int k = 0; k < SCAN_PER; k++)
-            if (i0 + k < n)
-                B.tile_order[atomicAdd(&s_hist[count_bucket(v[k])], 1u)] = i0 + k;
+            if (i0 + k < n) {
+                const uint32_t nb = bands(v[k]), tile = (i0 + k) * Q + queue;
+                const uint32_t at = atomicAdd(&s_hist[count_bucket(v[k] / nb)], nb);
+                if (nb == 1)
+                    *item_slot(B, at * Q + queue) = tile;
+                else
+                    for (uint32_t q = 0; q < SW_BANDS; q++)
+                        *item_slot(B, (at + q) * Q + queue) = tile | (q + 1) << SW_ITEM_BAND;
+            }
     }
 }
 
@@ -664,18 +706,20 @@ __global__ __launch_bounds__(256) void k_front(BatchDev B, const JobDev *__restr
 }
 
 // ----------------------------------------------------------- k_bin_fill
-// Block 0 writes the raster's claim order instead (the counts are final
-// once k_front has ended): dispatched first, it runs beside the fill, not
-// after it.  Block b > 0 fills for triangle block b - 1.
+// The first SW_RASTER_QUEUES blocks write the raster's claim order instead
+// (the counts are final once k_front has ended): dispatched first, they run
+// beside the fill, not after it.  Block b after them fills for triangle block
+// b - SW_RASTER_QUEUES.
 __global__ __launch_bounds__(256) void k_bin_fill(BatchDev B, const JobDev *__restrict__ jobs)
 {
-    if (blockIdx.x == 0) {
-        order_tiles<256>(B);
+    if (blockIdx.x < SW_RASTER_QUEUES) {
+        if (B.order)
+            order_tiles<256>(B, blockIdx.x);
         return;
     }
     // k_front placed every entry of a job unless one of its tiles
     // overflowed: then only the statistics, if asked for, are counted here
-    const uint32_t blk = blockIdx.x - 1;
+    const uint32_t blk = blockIdx.x - SW_RASTER_QUEUES;
     const int jidx = find_job<JT>(B, jobs, blk);
     const bool place = !B.fixed || B.ctr[SW_CTR_BIG0 + B.n_jobs + jidx] != 0;
     if (!place && !B.stats)
@@ -777,6 +821,15 @@ __device__ __forceinline__ float blur_factor(float z, float fdist, float fdepth,
     if (x >= rmax)
         return rmax;
     return 0.0f + rmax * x;
+}
+
+// What the depth-of-field pass reads of a pixel: whether its blur factor is
+// nonzero, and its radius in the bits above.
+__device__ __forceinline__ uint8_t dof_code(float z, float fdist, float fdepth, int rmax, const FDiv &by, bool fast)
+{
+    const float bf = blur_factor(z, fdist, fdepth, (float)rmax, by, fast);
+    const int radius = min(max(cvtt(bf), 0), rmax);   // bf is in [0, rmax] for finite inputs
+    return (uint8_t)((bf != 0.0f ? 1 : 0) | (radius << 1));
 }
 
 // ------------------------------------------------------------- k_raster
@@ -1347,12 +1400,28 @@ __device__ uint32_t shade_recorded(const JobDev &J, uint32_t seq, uint32_t tag, 
     return shade_from<GENERIC>(J, t, S, R, sp, u, oob);
 }
 
-template <int TW, int TH, bool GENERIC>
-__device__ __forceinline__ void raster_tile(const BatchDev &B, const JobDev *__restrict__ jobs, uint32_t g,
-                                            unsigned long long *keys, uint32_t *s_cnt, unsigned long long *slots)
+// Whether a tile's fragments record payload slots (put_slots, 24 bytes a
+// pixel): up to 64x32 pixels, whose 70 KB let two workgroups of 512 threads
+// on a CU.
+constexpr bool raster_slots(int tw, int th) { return tw * th <= 2048; }
+// Threads of a tile's workgroup.  Four waves fit on a SIMD at the raster's 128
+// registers whatever the workgroup's size; with more, smaller workgroups on a
+// CU one shades while another waits on its replay's loads and barriers
+// (32x32 tiles of the 999,698-triangle field at 3840x2160: 235 us with 256
+// threads, 290 with 512, 462 with 1,024).  Above 32x32 the slots' LDS allows
+// two workgroups, of 512.
+constexpr int raster_threads(int tw, int th) { return tw * th > 1024 ? 512 : 256; }
+
+template <int TW, int TH, int NT, bool GENERIC>
+__device__ __forceinline__ uint32_t raster_tile(const BatchDev &B, const JobDev *__restrict__ jobs, uint32_t item,
+                                                unsigned long long *keys, uint32_t *s_cnt,
+                                                unsigned long long *slots, uint32_t *claim)
 {
+    item = (uint32_t)__builtin_amdgcn_readfirstlane((int)item);   // the same in every lane
+    const uint32_t band = B.split == 0xFFFFFFFFu ? 0u : item >> SW_ITEM_BAND;
+    const uint32_t g = band ? item & ((1u << SW_ITEM_BAND) - 1u) : item;
     constexpr int NSLOT = TW * TH;
-    constexpr bool SLOTS = NSLOT <= 1024;   // as k_raster's
+    constexpr bool SLOTS = raster_slots(TW, TH);
     const int jidx = find_job<JTILE>(B, jobs, g);
     const JobDev &J = jobs[jidx];
     const int lt = (int)(g - J.tile_base);
@@ -1362,17 +1431,25 @@ __device__ __forceinline__ void raster_tile(const BatchDev &B, const JobDev *__r
     tr.y0 = J.V.vy + ty * TH;
     tr.x1 = min(tr.x0 + TW, J.V.vx + J.V.vw);
     tr.y1 = min(tr.y0 + TH, J.V.vy + J.V.vh);
+    // a band of the tile's rows: from here on a tile of its own, but for the
+    // entries (split tiles are at least 32 rows high)
+    int npix = TW * TH;
+    if (band) {
+        tr.y0 += (int)(band - 1u) * (TH / SW_BANDS);
+        tr.y1 = min(tr.y0 + TH / SW_BANDS, tr.y1);
+        npix = TW * (TH / SW_BANDS);
+    }
 
-    for (int i = threadIdx.x; i < TW * TH; i += 256)
+    for (int i = threadIdx.x; i < npix; i += NT)
         keys[i] = SW_KEY_EMPTY;
     __syncthreads();
 
     uint32_t frags = 0, nans = 0, oob = 0;
     // Replay the tile's binned triangles, then the job's big triangles whose
-    // rectangle touches this tile.  Up to 256 of them are cut into chunks of
+    // rectangle touches this tile.  Up to NT of them are cut into chunks of
     // rows, of about an equal number of pixels (from the screen bounding
     // boxes) and about as many as there are lanes, so that a few large
-    // triangles occupy every lane.  With more than 256, a lane takes a
+    // triangles occupy every lane.  With more, a lane takes a
     // triangle of its own, all rows, if it is plain and not one that covers
     // more than SW_LANE_PIXELS pixels of the tile, on which its lane would
     // spend several times what the others do; those are listed and cut up
@@ -1381,7 +1458,7 @@ __device__ __forceinline__ void raster_tile(const BatchDev &B, const JobDev *__r
     // of 330 entries with one large among them 65 us.  The 640x480 cube's
     // raster 45 -> 31 us, the 800x600 demo scene's 78 -> 47; chunks of at
     // least 16 or 32 pixels: 34 and 40 us for the cube.)
-    __shared__ uint32_t s_tri[256], s_rows[256], s_first[256], s_wsum[4], s_n;
+    __shared__ uint32_t s_tri[NT], s_rows[NT], s_first[NT], s_wsum[NT / 64], s_n;
     // The tile's entries: placed by k_front in its job's fixed layout
     // (every triangle whose rectangle holds the tile; marks are checked
     // here), or, when a tile of the job passed its capacity, by k_bin_fill
@@ -1456,7 +1533,7 @@ __device__ __forceinline__ void raster_tile(const BatchDev &B, const JobDev *__r
         return (tx >= (int)(r.x & 0xFFFF)) & (tx <= (int)(r.y & 0xFFFF)) & (ty >= (int)(r.x >> 16)) &
                (ty <= (int)(r.y >> 16));
     };
-    const bool many = entries > 256;
+    const bool many = entries > NT;
     uint32_t listed = entries;
     if (many) {
         if (threadIdx.x == 0)
@@ -1464,7 +1541,7 @@ __device__ __forceinline__ void raster_tile(const BatchDev &B, const JobDev *__r
         __syncthreads();
         auto list = [&](uint32_t t) {
             const uint32_t at = atomicAdd(&s_n, 1u);
-            if (at < 256u)
+            if (at < (uint32_t)NT)
                 s_tri[at] = t;
         };
         // The loads of an entry are a chain of three (entry, vertex ids,
@@ -1472,19 +1549,22 @@ __device__ __forceinline__ void raster_tile(const BatchDev &B, const JobDev *__r
         // their way while this one is replayed.
         const uint32_t flags = fixed ? SW_BIN_CHECK | SW_BIN_LARGE : 0u;
         if (threadIdx.x < nb) {
-            uint32_t e = threadIdx.x, k = ro(bins)[e], kn = ro(bins)[min(e + 256u, nb - 1u)];
+            uint32_t e = threadIdx.x, k = ro(bins)[e], kn = ro(bins)[min(e + NT, nb - 1u)];
             uint32_t t = k & ~flags, i0 = ro(W.tri)[3 * t], i1 = ro(W.tri)[3 * t + 1], i2 = ro(W.tri)[3 * t + 2];
-            for (;; e += 256) {
+            for (;; e += NT) {
                 PTri T;
                 T.a = tile_vertex(W, i0);
                 T.b = tile_vertex(W, i1);
                 T.c = tile_vertex(W, i2);
                 const uint32_t tn = kn & ~flags;
                 const uint32_t n0 = ro(W.tri)[3 * tn], n1 = ro(W.tri)[3 * tn + 1], n2 = ro(W.tri)[3 * tn + 2];
-                const uint32_t kn2 = ro(bins)[min(e + 512u, nb - 1u)];
+                const uint32_t kn2 = ro(bins)[min(e + 2u * NT, nb - 1u)];
                 const bool drawn = !(k & flags & SW_BIN_CHECK) ||
                                    ((ro(W.yes)[i0] != 0) & (ro(W.yes)[i1] != 0) & (ro(W.yes)[i2] != 0));
-                if (drawn) {
+                // (in a band most entries lie in other rows)
+                const bool here = !band || !(fmaxf(T.a.y, fmaxf(T.b.y, T.c.y)) <= (float)W.tr.y0 ||
+                                             fminf(T.a.y, fminf(T.b.y, T.c.y)) > (float)(W.tr.y1 - 1));
+                if (drawn && here) {
                     int ry0, ry1;
                     if (!is_plain(T) ||
                         ((k & flags & SW_BIN_LARGE) && rows_of(T, true, ry0, ry1) > SW_LANE_PIXELS))
@@ -1492,7 +1572,7 @@ __device__ __forceinline__ void raster_tile(const BatchDev &B, const JobDev *__r
                     else
                         plain_depth<TW, SLOTS>(W, T, t, i0, i1, i2, W.tr.y0, W.tr.y1, keys, slots, NSLOT, frags, nans);
                 }
-                if (e + 256 >= nb)
+                if (e + NT >= nb)
                     break;
                 k = kn;
                 t = tn;
@@ -1502,7 +1582,7 @@ __device__ __forceinline__ void raster_tile(const BatchDev &B, const JobDev *__r
                 kn = kn2;
             }
         }
-        for (uint32_t e = nb + threadIdx.x; e < entries; e += 256) {
+        for (uint32_t e = nb + threadIdx.x; e < entries; e += NT) {
             uint32_t t;
             bool check, large;
             if (entry(e, t, check, large) && marked(reread(jobs, jidx), t))
@@ -1511,11 +1591,11 @@ __device__ __forceinline__ void raster_tile(const BatchDev &B, const JobDev *__r
         __syncthreads();
         listed = s_n;
     }
-    // The listed triangles, 256 at a time.  More than 256 listed out of many
+    // The listed triangles, NT at a time.  More than NT listed out of many
     // are found again among the entries.
-    const bool again = many && listed > 256;
+    const bool again = many && listed > (uint32_t)NT;
     const uint32_t last = again ? entries : listed;
-    for (uint32_t base = 0; base < last; base += 256) {
+    for (uint32_t base = 0; base < last; base += NT) {
         uint32_t t = 0, area = 0;
         int ry0 = tr.y0, ry1 = tr.y0;
         if (base + threadIdx.x < last) {
@@ -1533,12 +1613,18 @@ __device__ __forceinline__ void raster_tile(const BatchDev &B, const JobDev *__r
                     area = 0;   // done above
             }
         }
+        auto block_total = [&] {
+            uint32_t n = 0;
+            for (int k = 0; k < NT / 64; k++)
+                n += s_wsum[k];
+            return n;
+        };
         // pixels of a chunk: an equal share of the list's for every lane
         const uint32_t sum = wave_sum(area);
         if (lane == 0)
             s_wsum[wave] = sum;
         __syncthreads();
-        const uint32_t per = max((s_wsum[0] + s_wsum[1] + s_wsum[2] + s_wsum[3]) / 256u, (uint32_t)SW_CHUNK_PIXELS);
+        const uint32_t per = max(block_total() / (uint32_t)NT, (uint32_t)SW_CHUNK_PIXELS);
         const uint32_t rows = (uint32_t)(ry1 - ry0);
         const uint32_t nch = area ? min(max(area / per, 1u), rows) : 0u;
         __syncthreads();   // s_wsum read, s_tri too
@@ -1552,12 +1638,12 @@ __device__ __forceinline__ void raster_tile(const BatchDev &B, const JobDev *__r
         uint32_t before = 0;
         for (int k = 0; k < wave; k++)
             before += s_wsum[k];
-        const uint32_t total = s_wsum[0] + s_wsum[1] + s_wsum[2] + s_wsum[3];
+        const uint32_t total = block_total();
         s_first[threadIdx.x] = before + incl - nch;
         __syncthreads();
-        for (uint32_t i = threadIdx.x; i < total; i += 256) {
+        for (uint32_t i = threadIdx.x; i < total; i += NT) {
             // the entry whose chunks contain item i: last k with s_first[k] <= i and chunks
-            int lo = 0, hi = 255;
+            int lo = 0, hi = NT - 1;
             while (lo < hi) {
                 const int mid = (lo + hi + 1) >> 1;
                 if (s_first[mid] <= i)
@@ -1580,13 +1666,19 @@ __device__ __forceinline__ void raster_tile(const BatchDev &B, const JobDev *__r
                 raster_depth_any(reread(jobs, jidx), tt, i0, i1, i2, tr, wy0, wy1, keys, TW, frags, nans,
                                  SLOTS ? slots : nullptr, NSLOT);
         }
-        __syncthreads();   // the LDS tables are rewritten by the next 256
+        __syncthreads();   // the LDS tables are rewritten by the next NT
     }
     __syncthreads();
 
+    // The claim of the next item is on its way while this one is shaded (a
+    // claim is a round trip to the memory side, 2-6 us with all workgroups
+    // claiming; between the items nothing of the workgroup ran meanwhile).
+    uint32_t next = 0;
+    if (claim && threadIdx.x == 0)
+        next = atomicAdd(claim, 1u);
     const JobDev &K = reread(jobs, jidx);
     const float maxz = __uint_as_float(SW_MAX_Z_BITS);
-    for (int i = threadIdx.x; i < TW * TH; i += 256) {
+    for (int i = threadIdx.x; i < npix; i += NT) {
         const int x = tr.x0 + (i % TW), y = tr.y0 + (i / TW);
         if (x >= tr.x1 || y >= tr.y1)
             continue;
@@ -1622,14 +1714,13 @@ __device__ __forceinline__ void raster_tile(const BatchDev &B, const JobDev *__r
     if (D.dofc) {
         const FDiv dof_by(D.fdepth - 1.0f);
         const bool dof_fast = D.fdepth - 1.0f >= 1.0f && D.fdepth - 1.0f <= 0x1p20f;
-        for (int i = threadIdx.x; i < TW * TH; i += 256) {
+        for (int i = threadIdx.x; i < npix; i += NT) {
             const int x = tr.x0 + (i % TW), y = tr.y0 + (i / TW);
             if (x >= tr.x1 || y >= tr.y1)
                 continue;
             const float z = __uint_as_float((uint32_t)(keys[i] >> 32));   // max_z where empty
-            const float bf = blur_factor(z, D.fdist, D.fdepth, (float)D.rmax, dof_by, dof_fast);
-            const int radius = min(max(cvtt(bf), 0), D.rmax);   // bf is in [0, rmax] for finite inputs
-            D.dofc[(int64_t)(y - D.V.vy) * D.V.vw + (x - D.V.vx)] = (uint8_t)((bf != 0.0f ? 1 : 0) | (radius << 1));
+            D.dofc[(int64_t)(y - D.V.vy) * D.V.vw + (x - D.V.vx)] =
+                dof_code(z, D.fdist, D.fdepth, D.rmax, dof_by, dof_fast);
         }
     }
     if (B.stats) {
@@ -1640,6 +1731,35 @@ __device__ __forceinline__ void raster_tile(const BatchDev &B, const JobDev *__r
         if (oob)
             atomicAdd(&s_cnt[2], oob);
     }
+    return next;
+}
+
+// A tile without entries: the clear alone (viewport.cpp:88-113) and the
+// depth-of-field code of max_z.
+template <int TW, int TH, int NT>
+__device__ __forceinline__ void fill_empty(const BatchDev &B, const JobDev *__restrict__ jobs, uint32_t g)
+{
+    const JobDev &J = jobs[find_job<JTILE>(B, jobs, g)];
+    const int lt = (int)(g - J.tile_base), tx = lt % J.tiles_x, ty = lt / J.tiles_x;
+    const float maxz = __uint_as_float(SW_MAX_Z_BITS);
+    uint8_t code = 0;
+    if (J.dofc) {
+        const FDiv by(J.fdepth - 1.0f);
+        const bool fast = J.fdepth - 1.0f >= 1.0f && J.fdepth - 1.0f <= 0x1p20f;
+        code = dof_code(maxz, J.fdist, J.fdepth, J.rmax, by, fast);
+    }
+    for (int i = threadIdx.x; i < TW * TH; i += NT) {
+        const int x = tx * TW + i % TW, y = ty * TH + i / TW;   // viewport-relative
+        if (x >= J.V.vw || y >= J.V.vh)
+            continue;
+        J.out_color[(int64_t)(y + J.V.vy - J.out_oy) * J.out_pitch + (x + J.V.vx - J.out_ox)] = 0u;
+        const int64_t zo = (int64_t)y * J.V.vw + x;
+        J.zbuf[zo] = maxz;
+        if (J.tid)
+            J.tid[zo] = 0xFFFFFFFFu;
+        if (J.dofc)
+            J.dofc[zo] = code;
+    }
 }
 
 // Persistent: each workgroup takes tiles from the batch's work queue until
@@ -1647,54 +1767,119 @@ __device__ __forceinline__ void raster_tile(const BatchDev &B, const JobDev *__r
 // At most 128 VGPRs, so four waves fit on each SIMD (512 registers a lane);
 // the shading path needs about that many and one more halves the overlap.
 template <int TW, int TH, bool GENERIC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_raster(BatchDev B,
-                                                                                     const JobDev *__restrict__ jobs)
+__global__ __launch_bounds__(raster_threads(TW, TH)) __attribute__((amdgpu_waves_per_eu(4))) void
+k_raster(BatchDev B, const JobDev *__restrict__ jobs)
 {
+    constexpr int NT = raster_threads(TW, TH);
+    constexpr uint32_t Q = SW_RASTER_QUEUES, NONE = 0xFFFFFFFFu;
     __shared__ unsigned long long keys[TW * TH];
-    // fragment payload slots (put_slots) for tiles of at most 32x32 pixels:
-    // 24 KB, which keeps four workgroups on a CU
-    constexpr bool SLOTS = TW * TH <= 1024;
-    __shared__ unsigned long long slots[SLOTS ? 3 * TW * TH : 1];
+    __shared__ unsigned long long slots[raster_slots(TW, TH) ? 3 * TW * TH : 1];
     __shared__ uint32_t s_cnt[3];
-    __shared__ uint32_t s_tile;
+    __shared__ uint32_t s_place;
     if (threadIdx.x < 3)
         s_cnt[threadIdx.x] = 0;
-    // Tiles come from SW_RASTER_QUEUES queues over the claim order
-    // (B.tile_order, largest bin counts first), queue k owning the places
-    // k, k + 8, k + 16, ... so that every queue runs from costly tiles to
-    // cheap ones, each counting on its own cache line: same-address atomics
-    // are serialised where they execute, so one shared queue would make every
-    // claim wait for all others.  A workgroup drains its home queue (block
-    // index mod 8), then the others in turn; a queue seen exhausted is never
-    // asked again, so every workgroup stops after at most n_tiles + 8 claims
-    // in total.
-    const uint32_t T = B.n_tiles, home = blockIdx.x % SW_RASTER_QUEUES;
-    uint32_t tried = 0;   // thread 0 only: queues found exhausted
-    for (;;) {
-        if (threadIdx.x == 0) {
-            uint32_t tile = 0xFFFFFFFFu;
-            while (tried < SW_RASTER_QUEUES) {
-                const uint32_t k = (home + tried) % SW_RASTER_QUEUES;
-                const uint32_t cnt = T > k ? (T - 1u - k) / SW_RASTER_QUEUES + 1u : 0u;   // places of queue k
-                uint32_t *q = &B.ctr[SW_CTR_QUEUE0 + 64 * k];
-                // counters only grow, so a stale read never skips a live queue
-                if (__hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < cnt) {
-                    const uint32_t i = atomicAdd(q, 1u);
-                    if (i < cnt) {
-                        tile = ro(B.tile_order)[k + SW_RASTER_QUEUES * i];
-                        break;
-                    }
-                }
-                tried++;
+    // Items come from SW_RASTER_QUEUES queues (order_tiles), each running from
+    // costly items to cheap ones and counting on its own cache line:
+    // same-address atomics are serialised where they execute, so one shared
+    // queue would make every claim wait for all others.  The first B.n_static
+    // workgroups, those that are resident together, begin with the places of
+    // their home queue (block index mod 8) that are theirs without a claim.
+    // A workgroup drains its home queue, its next claim on its way while the
+    // item before is shaded; then wave 0 reads the eight counters at once,
+    // one per lane (each read is a round trip to the memory side, and they
+    // are read only then: the claims of others wait behind them), and takes
+    // from the nearest queue that is not exhausted.  Counters only grow, so a
+    // queue seen exhausted stays so and every workgroup stops after at most
+    // n_items + 8 claims in total.
+    const uint32_t home = blockIdx.x % Q;
+    bool home_live = true;   // wave 0: the home queue was not seen exhausted
+    // wave 0: the next item's slot; `claimed`: this lane 0's count of its home
+    // queue, already taken
+    auto next_slot = [&](bool have, uint32_t claimed) {
+        // lane k: queue home + k, its items, and how many of them were given
+        // out without a claim (found again per claim: kept, they would cost
+        // the raster registers)
+        uint32_t lane = threadIdx.x;
+#if defined(__HIP_DEVICE_COMPILE__)
+        asm volatile("" : "+v"(lane));
+#endif
+        const uint32_t myq = (home + lane) % Q, cnt = B.ctr[SW_CTR_ITEMS + 2 * myq];
+        const uint32_t given = B.n_static > myq ? (B.n_static - 1u - myq) / Q + 1u : 0u;
+        uint32_t *const ctr = &B.ctr[SW_CTR_QUEUE0 + 64 * myq];
+        uint32_t slot = NONE;
+        if (home_live) {
+            if (threadIdx.x == 0) {
+                const uint32_t j = given + (have ? claimed : atomicAdd(ctr, 1u));
+                if (j < cnt)
+                    slot = j * Q + myq;
             }
-            s_tile = tile;
+            slot = (uint32_t)__builtin_amdgcn_readfirstlane((int)slot);
+            home_live = slot != NONE;
+        }
+        while (slot == NONE) {
+            const bool live = threadIdx.x < Q && given + __hip_atomic_load(ctr, __ATOMIC_RELAXED,
+                                                                           __HIP_MEMORY_SCOPE_AGENT) < cnt;
+            const uint64_t any = __ballot(live);
+            if (!any)
+                break;
+            const int l = __ffsll((unsigned long long)any) - 1;
+            if ((int)threadIdx.x == l) {
+                const uint32_t j = given + atomicAdd(ctr, 1u);
+                if (j < cnt)
+                    slot = j * Q + myq;
+            }
+            slot = __shfl(slot, l);
+        }
+        return slot;
+    };
+    uint32_t slot = NONE;
+    if (blockIdx.x < B.n_static) {
+        if (blockIdx.x / Q < (uint32_t)__builtin_amdgcn_readfirstlane((int)B.ctr[SW_CTR_ITEMS + 2 * home]))
+            slot = blockIdx.x;   // place blockIdx / 8 of queue blockIdx mod 8
+        else
+            home_live = false;
+    }
+    if (slot == NONE) {
+        if (threadIdx.x < 64) {
+            const uint32_t n = next_slot(false, 0);
+            if (threadIdx.x == 0)
+                s_place = n;
         }
         __syncthreads();
-        const uint32_t g = s_tile;
-        if (g == 0xFFFFFFFFu)
-            break;
-        raster_tile<TW, TH, GENERIC>(B, jobs, g, keys, s_cnt, slots);
-        __syncthreads();   // tile done with keys and s_tile before the next claim
+        slot = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_place);
+    }
+    while (slot != NONE) {
+        const bool ahead = home_live;
+        const uint32_t claimed = raster_tile<TW, TH, NT, GENERIC>(
+            B, jobs, *ro(item_slot(B, slot)), keys, s_cnt, slots, ahead ? &B.ctr[SW_CTR_QUEUE0 + 64 * home] : nullptr);
+        if (threadIdx.x < 64) {
+            const uint32_t n = next_slot(ahead, claimed);
+            if (threadIdx.x == 0)
+                s_place = n;
+        }
+        __syncthreads();   // also: the item is done with its keys
+        // (the next claim writes s_place behind the item's own barriers)
+        slot = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_place);
+    }
+    // The empty tiles of the home queue (of every queue where there are fewer
+    // workgroups than queues), SW_EMPTY_CLAIM at a time, by whoever is done: a
+    // claim each would take longer than their stores (of the 8,160 tiles of
+    // four 1920x1080 views of stacked clusters 5,881 are empty).
+    for (uint32_t q = home; q < (gridDim.x < Q ? home + Q : home + 1u); q++) {
+        const uint32_t k = q % Q;
+        const uint32_t T = (uint32_t)__builtin_amdgcn_readfirstlane((int)B.ctr[SW_CTR_ITEMS + 2 * k]),
+                       E = (uint32_t)__builtin_amdgcn_readfirstlane((int)B.ctr[SW_CTR_ITEMS + 2 * k + 1]);
+        while (E) {
+            __syncthreads();
+            if (threadIdx.x == 0)
+                s_place = atomicAdd(B.ctr + SW_CTR_EMPTYQ + 32 * k, (uint32_t)SW_EMPTY_CLAIM);
+            __syncthreads();
+            uint32_t c = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_place);
+            if (c >= E)
+                break;
+            for (const uint32_t end = min(c + SW_EMPTY_CLAIM, E); c < end; c++)
+                fill_empty<TW, TH, NT>(B, jobs, *ro(item_slot(B, (T + c) * Q + k)));
+        }
     }
     __syncthreads();
     if (B.stats && threadIdx.x == 0) {
@@ -2392,43 +2577,54 @@ hipError_t launch_front(const BatchDev &B, uint32_t blocks, hipStream_t s)
 }
 hipError_t launch_bin_fill(const BatchDev &B, uint32_t blocks, hipStream_t s, hipEvent_t done)
 {
-    // one more block than the fill needs: the first one writes the claim order
+    // SW_RASTER_QUEUES more blocks than the fill needs: the first ones write the claim order
     if (!B.n_tiles)
         return done ? hipEventRecord(done, s) : hipSuccess;
     if (done) {
         // the kernel's own completion signals `done`: no marker after it
-        hipExtLaunchKernelGGL(k_bin_fill, dim3(blocks + 1), dim3(256), 0, s, nullptr, done, 0, B, B.jobs);
+        hipExtLaunchKernelGGL(k_bin_fill, dim3(blocks + SW_RASTER_QUEUES), dim3(256), 0, s, nullptr, done, 0, B, B.jobs);
         return hipGetLastError();
     }
-    LAUNCH_CHECK(k_bin_fill, dim3(blocks + 1), dim3(256), 0, s, B, B.jobs);
+    LAUNCH_CHECK(k_bin_fill, dim3(blocks + SW_RASTER_QUEUES), dim3(256), 0, s, B, B.jobs);
+    return hipSuccess;
+}
+template <int TW, int TH, bool G>
+static hipError_t launch_raster_t(BatchDev B, uint32_t max_groups, uint32_t n_cus, hipStream_t s)
+{
+    constexpr int NT = raster_threads(TW, TH);
+    // max_groups counts groups of 256 threads
+    max_groups = std::max(1u, max_groups / (NT / 256));
+    // split tiles are several items (only k_bin_fill knows how many)
+    const uint64_t items = B.split == 0xFFFFFFFFu ? B.n_tiles : (uint64_t)B.n_tiles * SW_BANDS;
+    const uint32_t g = items < max_groups ? (uint32_t)items : max_groups;
+    B.n_static = std::min(g, n_cus * (1024 / NT));   // four waves a SIMD
+    LAUNCH_CHECK((k_raster<TW, TH, G>), dim3(g), dim3(NT), 0, s, B, B.jobs);
     return hipSuccess;
 }
 template <bool G>
-static hipError_t launch_raster_t(const BatchDev &B, int tw, int th, dim3 g, hipStream_t s)
+static hipError_t launch_raster_g(const BatchDev &B, int tw, int th, uint32_t max_groups, uint32_t n_cus, hipStream_t s)
 {
-    dim3 b(256);
     if (tw == 8 && th == 8)
-        LAUNCH_CHECK((k_raster<8, 8, G>), g, b, 0, s, B, B.jobs);
-    else if (tw == 16 && th == 16)
-        LAUNCH_CHECK((k_raster<16, 16, G>), g, b, 0, s, B, B.jobs);
-    else if (tw == 32 && th == 16)
-        LAUNCH_CHECK((k_raster<32, 16, G>), g, b, 0, s, B, B.jobs);
-    else if (tw == 32 && th == 32)
-        LAUNCH_CHECK((k_raster<32, 32, G>), g, b, 0, s, B, B.jobs);
-    else if (tw == 64 && th == 32)
-        LAUNCH_CHECK((k_raster<64, 32, G>), g, b, 0, s, B, B.jobs);
-    else if (tw == 64 && th == 64)
-        LAUNCH_CHECK((k_raster<64, 64, G>), g, b, 0, s, B, B.jobs);
-    else
-        return hipErrorInvalidValue;
-    return hipSuccess;
+        return launch_raster_t<8, 8, G>(B, max_groups, n_cus, s);
+    if (tw == 16 && th == 16)
+        return launch_raster_t<16, 16, G>(B, max_groups, n_cus, s);
+    if (tw == 32 && th == 16)
+        return launch_raster_t<32, 16, G>(B, max_groups, n_cus, s);
+    if (tw == 32 && th == 32)
+        return launch_raster_t<32, 32, G>(B, max_groups, n_cus, s);
+    if (tw == 64 && th == 32)
+        return launch_raster_t<64, 32, G>(B, max_groups, n_cus, s);
+    if (tw == 64 && th == 64)
+        return launch_raster_t<64, 64, G>(B, max_groups, n_cus, s);
+    return hipErrorInvalidValue;
 }
-hipError_t launch_raster(const BatchDev &B, int tw, int th, uint32_t max_groups, bool generic, hipStream_t s)
+hipError_t launch_raster(const BatchDev &B, int tw, int th, uint32_t max_groups, uint32_t n_cus, bool generic,
+                         hipStream_t s)
 {
     if (!B.n_tiles)
         return hipSuccess;
-    const dim3 g(B.n_tiles < max_groups ? B.n_tiles : max_groups);
-    return generic ? launch_raster_t<true>(B, tw, th, g, s) : launch_raster_t<false>(B, tw, th, g, s);
+    return generic ? launch_raster_g<true>(B, tw, th, max_groups, n_cus, s)
+                   : launch_raster_g<false>(B, tw, th, max_groups, n_cus, s);
 }
 
 hipError_t launch_layers(const BatchDev &B, bool generic, uint32_t pixels, hipStream_t s)

@@ -13,6 +13,7 @@ import pytest
 
 import oracle
 from swegl_amd.device import Context
+from swegl_amd.host import post_shader_depth_box
 
 from _helpers import compare, gpu_render
 from test_oracle_scene import flat_scene, view
@@ -77,6 +78,31 @@ def test_crowded_tiles(ctx, kind, entry):
             ctx.set_bin_limit(16)
         compare(got[0], want[0])
         assert got[0].stats["fragments"] == want[0].stats["fragments"]
+
+
+@pytest.mark.parametrize("w,h", [(40, 30), (97, 70), (700, 500)])
+@pytest.mark.parametrize("tile", [(16, 16), (32, 32), (64, 32), (64, 64)])
+def test_crowded_tiles_among_empty_ones(ctx, tile, w, h):
+    """9,000 triangles in one corner: more entries than a tile is rasterised
+    whole with (bands of its rows), queues without items, fewer workgroups
+    than queues, and tiles without entries, with depth of field on."""
+    rng = np.random.default_rng(w + tile[0])
+    s = flat_scene(triangles(rng, 9000, 0.02, (-0.6, 0.6), 0.04).tolist(), double_sided=True)
+    vp = view(w, h)
+    vp.set_post_shader(post_shader_depth_box(2.0, 1.5, vp, max_radius=4, taps="tap9"))
+    want = oracle.render(s, [vp])[0]
+    ctx.set_tile_auto(False)
+    ctx.set_tile(*tile)
+    try:
+        for groups in (1, 4):
+            ctx.set_raster_groups(groups)
+            got = gpu_render(ctx, s, [vp])[0]
+            compare(got, want, colour_tol=2)
+            assert got.stats["fragments"] == want.stats["fragments"]
+    finally:
+        ctx.set_tile_auto(True)
+        ctx.set_tile(32, 32)
+        ctx.set_raster_groups(4)
 
 
 def test_texture_coordinates_not_finite(ctx):
