@@ -99,7 +99,7 @@ struct ViewScratch {
 };
 
 struct swegl_scene {
-    DevBuf px, py, pz, nx, ny, nz, tu, tv, tri, prims, nodes, texels, texs, lights, world, nworld;
+    DevBuf px, py, pz, nx, ny, nz, tu, tv, tri, prims, nodes, texels, lights, world, nworld;
     uint32_t n_vertices = 0, n_tris = 0, n_prims = 0, n_lights = 0;
     bool no_material = false;   // some primitive has material_id -1
     std::vector<PrimDev> h_prims;
@@ -820,8 +820,26 @@ extern "C" int swegl_scene_upload(swegl_ctx *c, const swegl_scene_desc *d, swegl
     HIPCHK(hipSetDevice(c->device));
     std::unique_ptr<swegl_scene> s(new swegl_scene);
     // ---- validate and flatten primitives in draw order (nodes, then primitives)
-    std::vector<float> px, py, pz, nx, ny, nz, tu, tv;
-    std::vector<uint32_t> tri;
+    // the arrays' sizes first (what is out of range is refused below)
+    uint64_t nv = 0, nt = 0;
+    for (uint32_t ni = 0; ni < d->n_nodes; ni++) {
+        const swegl_node_desc &nd = d->nodes[ni];
+        if ((uint64_t)nd.first_primitive + nd.n_primitives > d->n_primitives)
+            break;
+        for (uint32_t k = 0; k < nd.n_primitives; k++) {
+            const swegl_primitive_desc &p = d->primitives[nd.first_primitive + k];
+            nv += p.n_vertices;
+            if (p.mode == SWEGL_TRIANGLES)
+                nt += p.n_indices / 3;
+            else if ((p.mode == SWEGL_TRIANGLE_STRIP || p.mode == SWEGL_TRIANGLE_FAN) && p.n_indices >= 3)
+                nt += p.n_indices - 2;
+        }
+    }
+    if (nv > 0x7FFFFFFFu || nt > 0x7FFFFFFFu)
+        return fail(SWEGL_EINVAL, "scene too large");
+    std::vector<float> px(nv), py(nv), pz(nv), nx(nv), ny(nv), nz(nv), tu(nv), tv(nv);
+    std::vector<uint32_t> tri(4 * nt);
+    size_t v_at = 0, t_at = 0;   // vertices and words of `tri` written
     for (uint32_t ni = 0; ni < d->n_nodes; ni++) {
         const swegl_node_desc &nd = d->nodes[ni];
         if ((uint64_t)nd.first_primitive + nd.n_primitives > d->n_primitives)
@@ -849,63 +867,66 @@ extern "C" int swegl_scene_upload(swegl_ctx *c, const swegl_scene_desc *d, swegl
                     return fail(SWEGL_EINVAL, "index %u out of range (%u vertices)", p.indices[i],
                                 p.n_vertices);
             PrimDev pd;
-            pd.first_vertex = (uint32_t)px.size();
+            pd.first_vertex = (uint32_t)v_at;
             pd.n_vertices = p.n_vertices;
-            pd.first_tri = (uint32_t)(tri.size() / 3);
+            pd.first_tri = (uint32_t)(t_at / 4);
             pd.node = ni;
             pd.tex = nomat ? -1 : m.texture_idx;
             pd.color = m.color;
             pd.double_sided = (!nomat && m.double_sided) ? 1 : 0;   // renderer.cpp:89-90
             const uint32_t base = pd.first_vertex;
-            for (uint32_t v = 0; v < p.n_vertices; v++) {
-                px.push_back(p.positions[3 * v]);
-                py.push_back(p.positions[3 * v + 1]);
-                pz.push_back(p.positions[3 * v + 2]);
-                nx.push_back(p.normals[3 * v]);
-                ny.push_back(p.normals[3 * v + 1]);
-                nz.push_back(p.normals[3 * v + 2]);
-                tu.push_back(p.tex_coords[2 * v]);
-                tv.push_back(p.tex_coords[2 * v + 1]);
+            for (uint32_t v = 0; v < p.n_vertices; v++, v_at++) {
+                px[v_at] = p.positions[3 * v];
+                py[v_at] = p.positions[3 * v + 1];
+                pz[v_at] = p.positions[3 * v + 2];
+                nx[v_at] = p.normals[3 * v];
+                ny[v_at] = p.normals[3 * v + 1];
+                nz[v_at] = p.normals[3 * v + 2];
+                tu[v_at] = p.tex_coords[2 * v];
+                tv[v_at] = p.tex_coords[2 * v + 1];
             }
             const uint32_t *I = p.indices;
             const size_t n = p.n_indices;
+            const uint32_t prim = (uint32_t)s->h_prims.size();
+            auto put = [&](uint32_t a, uint32_t b, uint32_t c) {
+                uint32_t *t = &tri[t_at];
+                t[0] = base + a;
+                t[1] = base + b;
+                t[2] = base + c;
+                t[3] = prim;
+                t_at += 4;
+            };
             // draw order and winding of renderer.cpp:197-229
             if (p.mode == SWEGL_TRIANGLE_STRIP)
-                for (size_t i = 2; i < n; i++) {
-                    tri.push_back(base + I[i - 2]);
-                    tri.push_back(base + I[i - 1 + (i & 1)]);
-                    tri.push_back(base + I[i - (i & 1)]);
-                }
+                for (size_t i = 2; i < n; i++)
+                    put(I[i - 2], I[i - 1 + (i & 1)], I[i - (i & 1)]);
             if (p.mode == SWEGL_TRIANGLE_FAN)
-                for (size_t i = 2; i < n; i++) {
-                    tri.push_back(base + I[0]);
-                    tri.push_back(base + I[i - 1]);
-                    tri.push_back(base + I[i]);
-                }
+                for (size_t i = 2; i < n; i++)
+                    put(I[0], I[i - 1], I[i]);
             if (p.mode == SWEGL_TRIANGLES)
-                for (size_t i = 2; i < n; i += 3) {
-                    tri.push_back(base + I[i - 2]);
-                    tri.push_back(base + I[i - 1]);
-                    tri.push_back(base + I[i]);
-                }
-            pd.n_tris = (uint32_t)(tri.size() / 3) - pd.first_tri;
+                for (size_t i = 2; i < n; i += 3)
+                    put(I[i - 2], I[i - 1], I[i]);
+            pd.n_tris = (uint32_t)(t_at / 4) - pd.first_tri;
             s->h_prims.push_back(pd);
         }
     }
-    if (px.size() > 0x7FFFFFFFu || tri.size() / 3 > 0x7FFFFFFFu)
-        return fail(SWEGL_EINVAL, "scene too large");
     s->n_vertices = (uint32_t)px.size();
-    s->n_tris = (uint32_t)(tri.size() / 3);
+    s->n_tris = (uint32_t)(tri.size() / 4);
     s->n_prims = (uint32_t)s->h_prims.size();
     // ---- textures
-    std::vector<TexDev> texs(std::max<uint32_t>(1, d->n_textures));
+    std::vector<uint64_t> first_texel(d->n_textures);
     uint64_t texels = 0;
     for (uint32_t i = 0; i < d->n_textures; i++) {
         const swegl_texture_desc &t = d->textures[i];
         if (!t.bitmap || t.width == 0 || t.height == 0 || t.width > 65536 || t.height > 65536)
             return fail(SWEGL_EINVAL, "texture %u is empty or too large", i);
-        texs[i] = TexDev{texels, (int32_t)t.width, (int32_t)t.height};
+        first_texel[i] = texels;
         texels += (uint64_t)t.width * t.height;
+    }
+    for (PrimDev &pd : s->h_prims) {
+        pd.texel = pd.tex >= 0 ? first_texel[pd.tex] : 0;
+        pd.tw = pd.tex >= 0 ? (int32_t)d->textures[pd.tex].width : 1;
+        pd.th = pd.tex >= 0 ? (int32_t)d->textures[pd.tex].height : 1;
     }
     int rc;
     const size_t V = std::max<size_t>(1, px.size());
@@ -913,9 +934,8 @@ extern "C" int swegl_scene_upload(swegl_ctx *c, const swegl_scene_desc *d, swegl
         (rc = s->nx.ensure(V * 4)) || (rc = s->ny.ensure(V * 4)) || (rc = s->nz.ensure(V * 4)) ||
         (rc = s->tu.ensure(V * 4)) || (rc = s->tv.ensure(V * 4)) ||
         (rc = s->world.ensure(V * 16)) || (rc = s->nworld.ensure(V * 16)) ||
-        (rc = s->tri.ensure(std::max<size_t>(3, tri.size()) * 4)) ||
+        (rc = s->tri.ensure(std::max<size_t>(4, tri.size()) * 4)) ||
         (rc = s->prims.ensure(std::max<size_t>(1, s->h_prims.size()) * sizeof(PrimDev))) ||
-        (rc = s->texs.ensure(texs.size() * sizeof(TexDev))) ||
         (rc = s->texels.ensure(std::max<uint64_t>(1, texels) * 4)))
         return rc;
     auto up = [&](DevBuf &b, const void *src, size_t bytes) -> int {
@@ -931,12 +951,11 @@ extern "C" int swegl_scene_upload(swegl_ctx *c, const swegl_scene_desc *d, swegl
         (rc = up(s->ny, ny.data(), ny.size() * 4)) || (rc = up(s->nz, nz.data(), nz.size() * 4)) ||
         (rc = up(s->tu, tu.data(), tu.size() * 4)) || (rc = up(s->tv, tv.data(), tv.size() * 4)) ||
         (rc = up(s->tri, tri.data(), tri.size() * 4)) ||
-        (rc = up(s->prims, s->h_prims.data(), s->h_prims.size() * sizeof(PrimDev))) ||
-        (rc = up(s->texs, texs.data(), texs.size() * sizeof(TexDev))))
+        (rc = up(s->prims, s->h_prims.data(), s->h_prims.size() * sizeof(PrimDev))))
         return rc;
     for (uint32_t i = 0; i < d->n_textures; i++) {
         const swegl_texture_desc &t = d->textures[i];
-        HIPCHK(hipMemcpyAsync(s->texels.as<uint32_t>() + texs[i].offset, t.bitmap,
+        HIPCHK(hipMemcpyAsync(s->texels.as<uint32_t>() + first_texel[i], t.bitmap,
                               (size_t)t.width * t.height * 4, hipMemcpyHostToDevice, c->stream));
     }
     if ((rc = scene_pose(c, s.get(), d)))
@@ -1184,11 +1203,10 @@ static int build_wave(swegl_ctx *c, Lane &L, const std::vector<JobIn> &jobs, Wav
         J.nz = s->nz.as<float>();
         J.tu = s->tu.as<float>();
         J.tv = s->tv.as<float>();
-        J.tri = s->tri.as<uint32_t>();
+        J.tri = s->tri.as<uint4>();
         J.prims = s->prims.as<PrimDev>();
         J.nodes = s->nodes.as<NodeDev>();
         J.texels = s->texels.as<uint32_t>();
-        J.texs = s->texs.as<TexDev>();
         J.lights = s->lights.as<Light4>();
         J.n_prims = s->n_prims;
         J.n_lights = s->n_lights;

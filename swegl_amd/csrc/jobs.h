@@ -4,14 +4,15 @@
 // HBM layout of a resident scene (SoA, all primitives concatenated in node
 // order, then primitive order):
 //   px,py,pz / nx,ny,nz / tu,tv : float[n_vertices]   mesh_vertex_t::v, normal, tex_coords
-//   tri                          : uint32[3*n_tris]    vertex ids per triangle in draw
-//                                                      order (strips/fans expanded with
-//                                                      the reference's winding)
-//   prims / nodes / texs         : small tables
+//   tri                          : uint4[n_tris]       vertex ids and primitive per
+//                                                      triangle in draw order (strips/fans
+//                                                      expanded with the reference's
+//                                                      winding): one load
+//   prims / nodes                : small tables
 //   texels                       : uint32 bitmaps of all textures, concatenated
 //   world, nworld                : float4[n_vertices]  v_world / normal_world for the
 //                                                      current node poses; .w holds the
-//                                                      texture coordinate u / v
+//                                                      texture coordinate u / v in texels
 // Per viewport job:
 //   ndc                          : float4[n_vertices]  frustum coordinates
 //   yes                          : uint8[n_vertices]   visibility marks
@@ -30,6 +31,8 @@ struct PrimDev {
     uint32_t first_tri, n_tris;
     uint32_t node;
     int32_t tex;           // texture index, or -1: 1x1 bitmap of `color`
+    uint64_t texel;        // the texture's first texel, its width and height (1 x 1 without)
+    int32_t tw, th;
     uint32_t color;        // material colour (default bitmap, pixel_shaders.cpp:290-294)
     int32_t double_sided;
 };
@@ -37,11 +40,6 @@ struct PrimDev {
 struct NodeDev {
     m34 M;     // original_to_world_matrix (rows 0..2)
     m34 RS;    // scale(rotation, scale) for normals (vertex_shaders.hpp:63)
-};
-
-struct TexDev {
-    uint64_t offset;   // into texels
-    int32_t w, h;
 };
 
 #define SW_MAX_DOF_RADIUS 16
@@ -64,11 +62,10 @@ __host__ __device__ inline uint32_t dof_blocks(int w, int h)
 struct JobDev {
     // ---- resident scene
     const float *px, *py, *pz, *nx, *ny, *nz, *tu, *tv;
-    const uint32_t *tri;
+    const uint4 *tri;
     const PrimDev *prims;
     const NodeDev *nodes;
     const uint32_t *texels;
-    const TexDev *texs;
     const Light4 *lights;
     uint32_t n_prims, n_lights, n_vertices, n_tris;
     float ambient, sun_I;

@@ -42,29 +42,11 @@ __device__ __forceinline__ int find_job(const BatchDev &B, const JobDev *__restr
     }
     return lo;
 }
-__device__ __forceinline__ int prim_of_vertex(const JobDev &J, uint32_t v)
+// Triangle t's vertex ids (x, y, z) and primitive (w).
+__device__ __forceinline__ uint4 tri_ids(const uint4 *tri, uint32_t t)
 {
-    int lo = 0, hi = (int)J.n_prims - 1;
-    while (lo < hi) {
-        int mid = (lo + hi + 1) >> 1;
-        if (ro(J.prims)[mid].first_vertex <= v)
-            lo = mid;
-        else
-            hi = mid - 1;
-    }
-    return lo;
-}
-__device__ __forceinline__ int prim_of_tri(const JobDev &J, uint32_t t)
-{
-    int lo = 0, hi = (int)J.n_prims - 1;
-    while (lo < hi) {
-        int mid = (lo + hi + 1) >> 1;
-        if (ro(J.prims)[mid].first_tri <= t)
-            lo = mid;
-        else
-            hi = mid - 1;
-    }
-    return lo;
+    const SW_RO uint32_t *q = ro((const uint32_t *)(tri + t));
+    return make_uint4(q[0], q[1], q[2], q[3]);
 }
 
 __device__ __forceinline__ f3 ld3(const float4 *a, uint32_t i)
@@ -143,10 +125,12 @@ __global__ __launch_bounds__(256) void k_world(WorldArgs W)
     const NodeDev &N = W.nodes[W.prims[lo].node];
     const f3 w = xform(N.M, f3{W.px[i], W.py[i], W.pz[i]});
     const f3 n = normal_world(N.RS, f3{W.nx[i], W.ny[i], W.nz[i]});
-    // the texture coordinates ride in the fourth lanes, so a shading lane
-    // gets a vertex's position, normal and coordinates in two loads
-    W.world[i] = make_float4(w.x, w.y, w.z, W.tu[i]);
-    W.nworld[i] = make_float4(n.x, n.y, n.z, W.tv[i]);
+    // the texture coordinates, in texels, ride in the fourth lanes, so a
+    // shading lane gets a vertex's position, normal and coordinates in two
+    // loads
+    const PrimDev &P = W.prims[lo];
+    W.world[i] = make_float4(w.x, w.y, w.z, W.tu[i] * (float)P.tw);
+    W.nworld[i] = make_float4(n.x, n.y, n.z, W.tv[i] * (float)P.th);
 }
 
 // ------------------------------------------------------------ k_vertex
@@ -179,7 +163,8 @@ __global__ __launch_bounds__(256) void k_vertex(BatchDev B, uint32_t w0, uint32_
 // draws a triangle only then).
 __device__ __forceinline__ bool marked(const JobDev &J, uint32_t t)
 {
-    return ro(J.yes)[ro(J.tri)[3 * t]] && ro(J.yes)[ro(J.tri)[3 * t + 1]] && ro(J.yes)[ro(J.tri)[3 * t + 2]];
+    const uint4 id = tri_ids(J.tri, t);
+    return (ro(J.yes)[id.x] != 0) & (ro(J.yes)[id.y] != 0) & (ro(J.yes)[id.z] != 0);
 }
 
 // ------------------------------------------------ fill_triangle on device
@@ -264,7 +249,8 @@ __device__ int tri_subs_v(const JobDev &J, uint32_t i0, uint32_t i1, uint32_t i2
 template <bool BINNED = false>
 __device__ __forceinline__ int tri_subs(const JobDev &J, uint32_t t, SubTri *out)
 {
-    return tri_subs_v<BINNED>(J, ro(J.tri)[3 * t], ro(J.tri)[3 * t + 1], ro(J.tri)[3 * t + 2], out);
+    const uint4 id = tri_ids(J.tri, t);
+    return tri_subs_v<BINNED>(J, id.x, id.y, id.z, out);
 }
 
 // Rows a sub-triangle's halves process, and a conservative column range.
@@ -616,10 +602,11 @@ __global__ __launch_bounds__(256) void k_front(BatchDev B, const JobDev *__restr
     bool self_marked = false;   // marked its own vertices: drawn whatever other triangles do
     bool large = false;         // may cover more than SW_LANE_PIXELS pixels of a tile
     if (t < J.n_tris) {
-        const uint32_t i0 = ro(J.tri)[3 * t], i1 = ro(J.tri)[3 * t + 1], i2 = ro(J.tri)[3 * t + 2];
+        const uint4 id = tri_ids(J.tri, t);
+        const uint32_t i0 = id.x, i1 = id.y, i2 = id.z;
         const f3 a = ld3(J.ndc, i0), b = ld3(J.ndc, i1), c = ld3(J.ndc, i2);
         if (inside_frustum(a, b, c) &&
-            (ro(J.prims)[prim_of_tri(J, t)].double_sided || cross_z_sign(b - a, c - a, 1))) {
+            (ro(J.prims)[id.w].double_sided || cross_z_sign(b - a, c - a, 1))) {
             J.yes[i0] = 1;
             J.yes[i1] = 1;
             J.yes[i2] = 1;
@@ -744,7 +731,8 @@ __global__ __launch_bounds__(256) void k_bin_fill(BatchDev B, const JobDev *__re
         }
         if (B.stats && m) {
             // drawn sub-triangles (fill_triangle_2 calls that find a scanline)
-            const uint32_t i0 = ro(J.tri)[3 * t], i1 = ro(J.tri)[3 * t + 1], i2 = ro(J.tri)[3 * t + 2];
+            const uint4 id = tri_ids(J.tri, t);
+            const uint32_t i0 = id.x, i1 = id.y, i2 = id.z;
             Extent E;
             bool exact;
             quick_extent(J, frustum_to_screen(J.V, ld3(J.ndc, i0)), frustum_to_screen(J.V, ld3(J.ndc, i1)),
@@ -1034,7 +1022,7 @@ __device__ __forceinline__ bool is_plain(const PTri &T)
 
 // What the replay reads of a tile's job, held for a whole tile.
 struct TileView {
-    const uint32_t *tri;
+    const uint4 *tri;
     const float4 *ndc;
     const uint8_t *yes;
     float m00, m03, m11, m13;
@@ -1208,196 +1196,194 @@ __device__ __forceinline__ void plain_depth(const TileView &W, const PTri &T, ui
     }
 }
 
-// Shading attributes of a sub-triangle vertex (v_world, normal_world, raw tex
-// coords, the last in the fourth lanes of world and nworld); clip vertices
-// are rebuilt as in renderer.cpp:290-297.
-__device__ void vertex_attr(const JobDev &J, const NodeDev &N, const SVert &v, f3 &w, f3 &n, f2 &t)
+// What the shading reads of a primitive.
+struct PrimView {
+    TexView X;        // its texture (pixel_shaders.cpp:288-302)
+    uint32_t color;   // its material's colour
+};
+__device__ __forceinline__ PrimView prim_view(const JobDev &J, const PrimDev &P)
 {
-    if (!v.clip) {
-        const float4 w4 = ro4(J.world, v.a), n4 = ro4(J.nworld, v.a);
-        w = f3{w4.x, w4.y, w4.z};
-        n = f3{n4.x, n4.y, n4.z};
-        t = f2{w4.w, n4.w};
-        return;
+    PrimView V{{nullptr, P.color, 1, 1}, P.color};
+    if (P.tex >= 0) {
+        V.X.p = J.texels + P.texel;
+        V.X.w = P.tw;
+        V.X.h = P.th;
     }
-    const float4 wa4 = ro4(J.world, v.a), wb4 = ro4(J.world, v.b);
-    const f3 wa = {wa4.x, wa4.y, wa4.z}, wb = {wb4.x, wb4.y, wb4.z};
-    w = wa + (wb - wa) * v.cut;
-    f2 ta = {wa4.w, ro4(J.nworld, v.a).w}, tb = {wb4.w, ro4(J.nworld, v.b).w};
-    t = ta + (tb - ta) * v.cut;
-    f3 na = {ro(J.nx)[v.a], ro(J.ny)[v.a], ro(J.nz)[v.a]}, nb = {ro(J.nx)[v.b], ro(J.ny)[v.b], ro(J.nz)[v.b]};
-    f3 nobj = (na.x == nb.x && na.y == nb.y && na.z == nb.z) ? na : normalize(na + (nb - na) * v.cut);
-    n = normal_world(N.RS, nobj);
+    return V;
+}
+// Primitive i's view; a scene of one primitive reads it with scalar loads.
+__device__ __forceinline__ PrimView prim_view(const JobDev &J, uint32_t i)
+{
+    if (J.n_prims == 1)
+        return prim_view(J, PrimDev(ro(J.prims)[0]));
+    return prim_view(J, PrimDev(ro(J.prims)[i]));
 }
 
-// The job's view of primitive P's texture (pixel_shaders.cpp:288-302).
-__device__ __forceinline__ TexView tex_view(const JobDev &J, const PrimDev &P)
+// A fragment to shade: the shading attributes of its sub-triangle's y-sorted
+// vertices (v_world, normal_world, texture coordinates in texels, the last in
+// the fourth lanes), its half and side order, the side progresses and its
+// progress u along the span.
+struct Frag {
+    float4 w[3], n[3];
+    bool lower, lr, inverted;
+    float pl, pr, u;
+    uint32_t prim;
+};
+
+// The attributes of sub-triangle vertex v; clip vertices are rebuilt as in
+// renderer.cpp:290-297.
+__device__ void vertex_attr(const JobDev &J, const PrimDev &P, const SVert &v, float4 &w, float4 &n)
 {
-    TexView X{nullptr, P.color, 1, 1};
-    if (P.tex >= 0) {
-        const TexDev T = ro(J.texs)[P.tex];
-        X.p = J.texels + T.offset;
-        X.w = T.w;
-        X.h = T.h;
+    if (!v.clip) {
+        w = ro4(J.world, v.a);
+        n = ro4(J.nworld, v.a);
+        return;
     }
-    return X;
+    const f3 wa = ld3(J.world, v.a), wb = ld3(J.world, v.b);
+    const f3 wc = wa + (wb - wa) * v.cut;
+    const f2 ta = {ro(J.tu)[v.a], ro(J.tv)[v.a]}, tb = {ro(J.tu)[v.b], ro(J.tv)[v.b]};
+    const f2 tc = ta + (tb - ta) * v.cut;
+    f3 na = {ro(J.nx)[v.a], ro(J.ny)[v.a], ro(J.nz)[v.a]}, nb = {ro(J.nx)[v.b], ro(J.ny)[v.b], ro(J.nz)[v.b]};
+    f3 nobj = (na.x == nb.x && na.y == nb.y && na.z == nb.z) ? na : normalize(na + (nb - na) * v.cut);
+    const NodeDev N = ro(J.nodes)[P.node];
+    const f3 nc = normal_world(N.RS, nobj);
+    w = make_float4(wc.x, wc.y, wc.z, tc.x * (float)P.tw);
+    n = make_float4(nc.x, nc.y, nc.z, tc.y * (float)P.th);
+}
+// A fragment from its replayed setup, row and span.
+__device__ __forceinline__ void frag_of(const JobDev &J, uint32_t t, const Setup &S, const Row &R, const Span &sp,
+                                        float u, Frag &F)
+{
+    F.prim = tri_ids(J.tri, t).w;
+    const PrimDev P = ro(J.prims)[F.prim];
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+        vertex_attr(J, P, S.v[k], F.w[k], F.n[k]);
+    F.lower = R.lower;
+    F.lr = R.lr;
+    F.inverted = S.inverted;
+    F.pl = sp.pl;
+    F.pr = sp.pr;
+    F.u = u;
+}
+
+// The texture part of a shader kind: 0 the material colour, 1 nearest, 2
+// bilinear.
+__device__ __forceinline__ int texture_kind(int k)
+{
+    return (k == 1 || k == 3 || k == 7) ? 2 : (k == 2 || k == 4 || k == 6) ? 1 : 0;
+}
+
+// The colour of a fragment before lighting: the material colour, nearest
+// texel or bilinear texel of the shader's texture part.  Its alpha is the
+// fragment's alpha for every shader whose light part only scales b, g, r
+// (a10, pixel_shaders.hpp:121-179) -- all but the light-only ones.
+template <bool GENERIC>
+__device__ __forceinline__ uint32_t frag_texture(const JobDev &J, const Frag &F, const RowEnds &E, uint32_t &oob)
+{
+    const int tk = GENERIC ? texture_kind(J.shader) : 2;
+    const PrimView P = prim_view(J, F.prim);
+    if (tk == 0)
+        return P.color;
+    const float su = E.along(F.u);
+    const f2 tc = {RowVal(E, F.w[0].w, F.w[1].w, F.w[2].w).at(su), RowVal(E, F.n[0].w, F.n[1].w, F.n[2].w).at(su)};
+    return tk == 1 ? nearest(P.X, tc) : bilinear(P.X, tc, oob);
 }
 
 // GENERIC: the job's shader is any SWEGL_SHADER_* kind, decoded into a light
-// part (0 none, 1 flat, 2 phong) and a texture part (0 the material colour,
-// 1 nearest, 2 bilinear); otherwise it is SWEGL_SHADER_PHONG_BILINEAR, the
-// kernel variant the common case runs without the other branches.
-// Shading of triangle t's fragment with progress u on the row and span
-// already set up (S, R, sp).
+// part (0 none, 1 flat, 2 phong) and a texture part; otherwise it is
+// SWEGL_SHADER_PHONG_BILINEAR, the kernel variant the common case runs without
+// the other branches.
 template <bool GENERIC>
-__device__ uint32_t shade_from(const JobDev &J, uint32_t t, const Setup &S, const Row &R, const Span &sp,
-                               float u, uint32_t &oob)
+__device__ __forceinline__ uint32_t shade_frag(const JobDev &J, const Frag &F, uint32_t &oob)
 {
-    int lk = 2, tk = 2;
+    int lk = 2;
     bool combined = true;
     if (GENERIC) {
         const int k = J.shader;
         lk = (k == 1 || k == 2 || k == 9) ? 2 : (k == 3 || k == 4 || k == 8) ? 1 : 0;
-        tk = (k == 1 || k == 3 || k == 7) ? 2 : (k == 2 || k == 4 || k == 6) ? 1 : 0;
         combined = k >= 1 && k <= 4;
     }
-    const PrimDev P = ro(J.prims)[prim_of_tri(J, t)];
-    const NodeDev N = ro(J.nodes)[P.node];
-    const TexView X = tex_view(J, P);
-    const int tw = X.w, th = X.h;
-    TriAttr A;
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        f3 w, n;
-        f2 tc;
-        vertex_attr(J, N, S.v[k], w, n, tc);
-        A.w[k] = w;
-        A.n[k] = S.inverted ? neg(n) : n;
-        A.t[k] = f2{tc.x * (float)tw, tc.y * (float)th};
-    }
-    ScanShade SS = prepare_scanline(A, R.lower, R.lr, sp.pl, sp.pr);
-    if (!GENERIC) {
-        uint32_t color = bilinear(X, SS.t_left + SS.t_dir * u, oob);
-        f3 center = SS.v + SS.vdir * u;
-        f3 normal = normalize(SS.n + SS.ndir * u);
-        int32_t light = phong(center, normal, J.V.cam, J.ambient, J.sun, J.sun_I, J.lights, (int)J.n_lights);
-        return combine(color, light);
-    }
-    uint32_t color = P.color;   // pixel_shader_t::color (default material for material_id -1)
-    if (tk == 1)
-        color = nearest(X, SS.t_left + SS.t_dir * u);
-    else if (tk == 2)
-        color = bilinear(X, SS.t_left + SS.t_dir * u, oob);
-    if (lk == 0)
+    const RowEnds E(F.lower, F.lr, F.pl, F.pr);
+    const uint32_t color = frag_texture<GENERIC>(J, F, E, oob);
+    if (GENERIC && lk == 0)
         return color;
     int32_t light;
-    if (lk == 1) {
-        light = flat_light(A.w[0], A.w[1], A.w[2], S.inverted, J.V.cam, J.ambient, J.sun, J.sun_I, J.lights,
-                           (int)J.n_lights);
+    if (GENERIC && lk == 1) {
+        light = flat_light(f3{F.w[0].x, F.w[0].y, F.w[0].z}, f3{F.w[1].x, F.w[1].y, F.w[1].z},
+                           f3{F.w[2].x, F.w[2].y, F.w[2].z}, F.inverted, J.V.cam, J.ambient, J.sun, J.sun_I,
+                           J.lights, (int)J.n_lights);
     } else {
-        f3 center = SS.v + SS.vdir * u;
-        f3 normal = normalize(SS.n + SS.ndir * u);
-        light = phong(center, normal, J.V.cam, J.ambient, J.sun, J.sun_I, J.lights, (int)J.n_lights);
+        const float su = E.along(F.u);
+        const f3 center = {RowVal(E, F.w[0].x, F.w[1].x, F.w[2].x).at(su),
+                           RowVal(E, F.w[0].y, F.w[1].y, F.w[2].y).at(su),
+                           RowVal(E, F.w[0].z, F.w[1].z, F.w[2].z).at(su)};
+        f3 normal = {RowVal(E, F.n[0].x, F.n[1].x, F.n[2].x).at(su), RowVal(E, F.n[0].y, F.n[1].y, F.n[2].y).at(su),
+                     RowVal(E, F.n[0].z, F.n[1].z, F.n[2].z).at(su)};
+        // an inverted triangle's vertex normals are negated
+        // (pixel_shaders.cpp:88-110): the interpolation only adds, subtracts
+        // and scales them, so the sign is as well applied at its end
+        if (F.inverted)
+            normal = neg(normal);
+        light = phong(center, normalize(normal), J.V.cam, J.ambient, J.sun, J.sun_I, J.lights, (int)J.n_lights);
     }
     return combined ? combine(color, light) : (uint32_t)light;
 }
 
-// The colour of triangle t's fragment before lighting: the material colour,
-// nearest texel or bilinear texel of the shader's texture part.  Its alpha
-// is the fragment's alpha for every shader whose light part only scales
-// b, g, r (a10, pixel_shaders.hpp:121-179) -- all but the light-only ones.
-template <bool GENERIC>
-__device__ uint32_t texture_from(const JobDev &J, uint32_t t, const Setup &S, const Row &R, const Span &sp,
-                                 float u, uint32_t &oob)
-{
-    int tk = 2;
-    if (GENERIC) {
-        const int k = J.shader;
-        tk = (k == 1 || k == 3 || k == 7) ? 2 : (k == 2 || k == 4 || k == 6) ? 1 : 0;
-    }
-    const PrimDev P = ro(J.prims)[prim_of_tri(J, t)];
-    if (tk == 0)
-        return P.color;
-    const NodeDev N = ro(J.nodes)[P.node];
-    const TexView X = tex_view(J, P);
-    const int tw = X.w, th = X.h;
-    TriAttr A;
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        f3 w, n;
-        f2 tc;
-        vertex_attr(J, N, S.v[k], w, n, tc);
-        A.w[k] = w;
-        A.n[k] = n;
-        A.t[k] = f2{tc.x * (float)tw, tc.y * (float)th};
-    }
-    ScanShade SS = prepare_scanline(A, R.lower, R.lr, sp.pl, sp.pr);
-    if (tk == 1)
-        return nearest(X, SS.t_left + SS.t_dir * u);
-    return bilinear(X, SS.t_left + SS.t_dir * u, oob);
-}
-
-// Shading of the winning draw sequence seq at pixel (x, y): the sub-triangle,
-// row and span re-derived by the same replay that produced the winner.
-template <bool GENERIC>
-__device__ uint32_t shade_pixel(const JobDev &J, uint32_t seq, int x, int y, uint32_t &oob)
+// The fragment of the winning draw sequence seq at pixel (x, y): the
+// sub-triangle, row and span re-derived by the same replay that produced the
+// winner, so every step succeeds; false only for a corrupted key.
+__device__ __forceinline__ bool frag_replayed(const JobDev &J, uint32_t seq, int x, int y, Frag &F)
 {
     const uint32_t t = seq >> 1, s = seq & 1u;
     SubTri st[2];
     Setup S;
     Row R;
     Span sp;
-    // The winner was produced by this very replay, so every step below
-    // succeeds; the guards only keep a corrupted key from looping.
     if ((int)s >= tri_subs<true>(J, t, st))
-        return 0u;
+        return false;
     SubTri one = st[0];   // a copy, not a runtime index: st stays in registers
     if (s)
         one = st[1];
     if (!setup_subtri(one, J.V, S, y) || !row_state(S, y, R) || !span_of(R, J.V, sp) || x < sp.x1 || x >= sp.x2)
-        return 0u;
+        return false;
     Interp q = sp.q;
     q.steps(x - sp.x1);
-    return shade_from<GENERIC>(J, t, S, R, sp, q.u(), oob);
+    frag_of(J, t, S, R, sp, q.u(), F);
+    return true;
+}
+template <bool GENERIC>
+__device__ uint32_t shade_pixel(const JobDev &J, uint32_t seq, int x, int y, uint32_t &oob)
+{
+    Frag F;
+    return frag_replayed(J, seq, x, y, F) ? shade_frag<GENERIC>(J, F, oob) : 0u;
 }
 
-// Shading of the winning sequence seq from its recorded payload (put_slots):
-// the sub-triangle's vertices in fill_triangle_2's order, the half and side
-// order, the side progresses and the span progress u.
-template <bool GENERIC>
-__device__ uint32_t shade_recorded(const JobDev &J, uint32_t seq, uint32_t tag, float u, float pl, float pr,
-                                   uint32_t &oob)
+// The fragment of an unclipped triangle from its recorded payload
+// (put_slots): the vertices in fill_triangle_2's order, the half and side
+// order, the side progresses and the span progress u.  id: the triangle's
+// vertices and primitive.
+__device__ __forceinline__ void frag_recorded(const JobDev &J, uint4 id, uint32_t tag, float u, float pl, float pr,
+                                              Frag &F)
 {
-    const uint32_t t = seq >> 1, s = seq & 1u, code = (tag >> 25) & 31u, perm = code & 15u;
-    Setup S;
-    if (perm < 9u) {
-        // fill_triangle_2's vertex order, recorded: no z- or y-sort to redo
-        const uint32_t id[3] = {ro(J.tri)[3 * t], ro(J.tri)[3 * t + 1], ro(J.tri)[3 * t + 2]};
-        const uint32_t p0 = perm / 3u, p1 = perm % 3u, p2 = 3u - p0 - p1;
-        const uint32_t ids[3] = {id[p0], id[p1], id[p2]};
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            S.v[k].a = S.v[k].b = ids[k];
-            S.v[k].cut = 0.0f;
-            S.v[k].clip = 0;
-        }
-        S.inverted = (code & 16u) != 0;
-    } else {
-        SubTri st[2];
-        if ((int)s >= tri_subs<true>(J, t, st))
-            return 0u;   // not reached: the winner came out of this sub-triangle
-        SubTri one = st[0];
-        if (s)
-            one = st[1];
-        sort_subtri(one, S);
-    }
-    Row R;
-    R.lower = (tag >> 30) & 1u;
-    R.lr = (tag >> 31) & 1u;
-    Span sp;
-    sp.pl = pl;
-    sp.pr = pr;
-    return shade_from<GENERIC>(J, t, S, R, sp, u, oob);
+    const uint32_t code = (tag >> 25) & 31u, perm = code & 15u;
+    // (p0, p1) of 3 * p0 + p1; p2 is the third
+    const bool a0 = perm < 3u, b0 = perm < 6u, a1 = perm == 3u || perm == 6u, b1 = perm == 1u || perm == 7u;
+    const uint32_t i0 = a0 ? id.x : b0 ? id.y : id.z, i1 = a1 ? id.x : b1 ? id.y : id.z;
+    const uint32_t i2 = id.x ^ id.y ^ id.z ^ i0 ^ i1;   // three different ids
+    F.w[0] = ro4(J.world, i0);
+    F.n[0] = ro4(J.nworld, i0);
+    F.w[1] = ro4(J.world, i1);
+    F.n[1] = ro4(J.nworld, i1);
+    F.w[2] = ro4(J.world, i2);
+    F.n[2] = ro4(J.nworld, i2);
+    F.lower = (tag >> 30) & 1u;
+    F.lr = (tag >> 31) & 1u;
+    F.inverted = (code & 16u) != 0;
+    F.pl = pl;
+    F.pr = pr;
+    F.u = u;
+    F.prim = id.w;
 }
 
 // Whether a tile's fragments record payload slots (put_slots, 24 bytes a
@@ -1490,9 +1476,10 @@ __device__ __forceinline__ uint32_t raster_tile(const BatchDev &B, const JobDev 
     // Triangle t's vertices, and whether it is drawn: `check`, its marks are
     // still to be looked up.
     auto load = [&](uint32_t t, bool check, uint32_t &i0, uint32_t &i1, uint32_t &i2, PTri &T) {
-        i0 = ro(W.tri)[3 * t];
-        i1 = ro(W.tri)[3 * t + 1];
-        i2 = ro(W.tri)[3 * t + 2];
+        const uint4 id = tri_ids(W.tri, t);
+        i0 = id.x;
+        i1 = id.y;
+        i2 = id.z;
         T.a = tile_vertex(W, i0);
         T.b = tile_vertex(W, i1);
         T.c = tile_vertex(W, i2);
@@ -1550,14 +1537,17 @@ __device__ __forceinline__ uint32_t raster_tile(const BatchDev &B, const JobDev 
         const uint32_t flags = fixed ? SW_BIN_CHECK | SW_BIN_LARGE : 0u;
         if (threadIdx.x < nb) {
             uint32_t e = threadIdx.x, k = ro(bins)[e], kn = ro(bins)[min(e + NT, nb - 1u)];
-            uint32_t t = k & ~flags, i0 = ro(W.tri)[3 * t], i1 = ro(W.tri)[3 * t + 1], i2 = ro(W.tri)[3 * t + 2];
+            uint32_t t = k & ~flags;
+            const uint4 id0 = tri_ids(W.tri, t);
+            uint32_t i0 = id0.x, i1 = id0.y, i2 = id0.z;
             for (;; e += NT) {
                 PTri T;
                 T.a = tile_vertex(W, i0);
                 T.b = tile_vertex(W, i1);
                 T.c = tile_vertex(W, i2);
                 const uint32_t tn = kn & ~flags;
-                const uint32_t n0 = ro(W.tri)[3 * tn], n1 = ro(W.tri)[3 * tn + 1], n2 = ro(W.tri)[3 * tn + 2];
+                const uint4 idn = tri_ids(W.tri, tn);
+                const uint32_t n0 = idn.x, n1 = idn.y, n2 = idn.z;
                 const uint32_t kn2 = ro(bins)[min(e + 2u * NT, nb - 1u)];
                 const bool drawn = !(k & flags & SW_BIN_CHECK) ||
                                    ((ro(W.yes)[i0] != 0) & (ro(W.yes)[i1] != 0) & (ro(W.yes)[i2] != 0));
@@ -1678,35 +1668,46 @@ __device__ __forceinline__ uint32_t raster_tile(const BatchDev &B, const JobDev 
         next = atomicAdd(claim, 1u);
     const JobDev &K = reread(jobs, jidx);
     const float maxz = __uint_as_float(SW_MAX_Z_BITS);
+    // the winner's vertex ids are loaded one pixel ahead
+    auto winner_ids = [&](int i) {
+        const unsigned long long k = i < npix ? keys[i] : SW_KEY_EMPTY;
+        return k != SW_KEY_EMPTY ? tri_ids(K.tri, (uint32_t)k >> 1) : make_uint4(0, 0, 0, 0);
+    };
+    uint4 id = winner_ids(threadIdx.x);
     for (int i = threadIdx.x; i < npix; i += NT) {
+        const uint4 id_next = winner_ids(i + NT);
         const int x = tr.x0 + (i % TW), y = tr.y0 + (i / TW);
-        if (x >= tr.x1 || y >= tr.y1)
-            continue;
-        const unsigned long long k = keys[i];
-        uint32_t color = 0;
-        float z = maxz;
-        uint32_t seq = 0xFFFFFFFFu;
-        if (k != SW_KEY_EMPTY) {
-            seq = (uint32_t)k;
-            z = __uint_as_float((uint32_t)(k >> 32));
-            bool done = false;
-            if (SLOTS) {
-                const unsigned long long a = slots[i], b = slots[NSLOT + i], c = slots[2 * NSLOT + i];
-                const uint32_t tag = (uint32_t)(a >> 32);
-                if (tag == (uint32_t)(b >> 32) && tag == (uint32_t)(c >> 32) && (tag & SW_SLOT_SEQ) == seq) {
-                    color = shade_recorded<GENERIC>(K, seq, tag, __uint_as_float((uint32_t)a),
-                                                    __uint_as_float((uint32_t)b), __uint_as_float((uint32_t)c), oob);
-                    done = true;
+        if (x < tr.x1 && y < tr.y1) {
+            const unsigned long long k = keys[i];
+            uint32_t color = 0;
+            float z = maxz;
+            uint32_t seq = 0xFFFFFFFFu;
+            if (k != SW_KEY_EMPTY) {
+                seq = (uint32_t)k;
+                z = __uint_as_float((uint32_t)(k >> 32));
+                Frag F;
+                bool have = false;
+                if (SLOTS) {
+                    const unsigned long long a = slots[i], b = slots[NSLOT + i], c = slots[2 * NSLOT + i];
+                    const uint32_t tag = (uint32_t)(a >> 32);
+                    have = (tag == (uint32_t)(b >> 32)) & (tag == (uint32_t)(c >> 32)) & ((tag & SW_SLOT_SEQ) == seq) &
+                           ((tag >> 25 & 15u) < 9u);
+                    if (have)
+                        frag_recorded(K, id, tag, __uint_as_float((uint32_t)a), __uint_as_float((uint32_t)b),
+                                      __uint_as_float((uint32_t)c), F);
                 }
+                if (!have)
+                    have = frag_replayed(K, seq, x, y, F);
+                if (have)
+                    color = shade_frag<GENERIC>(K, F, oob);
             }
-            if (!done)
-                color = shade_pixel<GENERIC>(K, seq, x, y, oob);
+            K.out_color[(int64_t)(y - K.out_oy) * K.out_pitch + (x - K.out_ox)] = color;
+            const int64_t zo = (int64_t)(y - K.V.vy) * K.V.vw + (x - K.V.vx);
+            K.zbuf[zo] = z;
+            if (K.tid)
+                K.tid[zo] = seq;
         }
-        K.out_color[(int64_t)(y - K.out_oy) * K.out_pitch + (x - K.out_ox)] = color;
-        const int64_t zo = (int64_t)(y - K.V.vy) * K.V.vw + (x - K.V.vx);
-        K.zbuf[zo] = z;
-        if (K.tid)
-            K.tid[zo] = seq;
+        id = id_next;
     }
     // The depth-of-field pass reads this code instead of z.  A loop of its
     // own keeps its registers out of the shading loop's peak.
@@ -2037,42 +2038,34 @@ __device__ __forceinline__ uint32_t blend_colors(uint32_t back, uint32_t front)
 }
 
 // The fragments of triangle t's unclipped sub-triangle over the tile's rows
-// [ty0, ty0 + TH) and columns [tx0, tx0 + TW): the same row walk and span
+// [row0, row1) and columns [tx0, tx0 + TW): the same row walk and span
 // stepping as raster_depth (renderer.cpp:462-558), writing each covered
 // pixel's depth to z[py * TW + px] and its bit to the returned mask.  With
 // `opaque`, also the bit of every covered pixel whose texture-part colour
-// (texture_from: material colour, nearest or bilinear texel) has alpha 255,
+// (frag_texture: material colour, nearest or bilinear texel) has alpha 255,
 // from the same row and span state a re-derivation for that pixel gives.
 template <bool GENERIC>
-__device__ uint64_t layer_walk(const JobDev &J, uint32_t t, const SubTri &st, int tx0, int ty0, float *z,
-                               uint64_t *opaque)
+__device__ uint64_t layer_walk(const JobDev &J, uint32_t t, const SubTri &st, int tx0, int ty0, int row0, int row1,
+                               float *z, uint64_t *opaque)
 {
-    constexpr int TW = SW_LAYER_TW, TH = SW_LAYER_TH;
+    constexpr int TW = SW_LAYER_TW;
     Setup S;
     if (!setup_subtri(st, J.V, S))
         return 0ull;
-    // texture part of the colour (texture_from)
-    int tk = 2;
-    if (GENERIC) {
-        const int k = J.shader;
-        tk = (k == 1 || k == 3 || k == 7) ? 2 : (k == 2 || k == 4 || k == 6) ? 1 : 0;
-    }
-    const PrimDev P = ro(J.prims)[prim_of_tri(J, t)];
-    TexView X{nullptr, P.color, 1, 1};
-    TriAttr A;
+    // texture part of the colour (frag_texture)
+    const int tk = GENERIC ? texture_kind(J.shader) : 2;
+    const PrimView P = prim_view(J, tri_ids(J.tri, t).w);
+    const TexView &X = P.X;
+    f2 tc[3];
     uint64_t opq = 0ull;
     const bool textured = opaque != nullptr && tk != 0;
     if (textured) {
-        X = tex_view(J, P);
 #pragma unroll
-        for (int k = 0; k < 3; k++) {
-            A.w[k] = f3{0.0f, 0.0f, 0.0f};
-            A.n[k] = f3{0.0f, 0.0f, 0.0f};
-            A.t[k] = f2{ro4(J.world, S.v[k].a).w * (float)X.w, ro4(J.nworld, S.v[k].a).w * (float)X.h};
-        }
+        for (int k = 0; k < 3; k++)
+            tc[k] = f2{ro4(J.world, S.v[k].a).w, ro4(J.nworld, S.v[k].a).w};
     }
     const bool flat_opaque = (P.color >> 24) == 255;   // tk == 0: the material colour
-    const int wy0 = ty0, wy1 = min(ty0 + TH, J.V.vy + J.V.vh), wx1 = min(tx0 + TW, J.V.vx + J.V.vw);
+    const int wy0 = ty0 + row0, wy1 = min(ty0 + row1, J.V.vy + J.V.vh), wx1 = min(tx0 + TW, J.V.vx + J.V.vw);
     uint64_t mask = 0ull;
     walk_rows(S, wy0, wy1, [&](int y, const Row &R) {
         Span sp;
@@ -2083,9 +2076,12 @@ __device__ uint64_t layer_walk(const JobDev &J, uint32_t t, const SubTri &st, in
             return;
         Interp q = sp.q;
         q.steps(xa - sp.x1);
-        ScanShade SS;
-        if (textured)
-            SS = prepare_scanline(A, R.lower, R.lr, sp.pl, sp.pr);
+        const RowEnds E(R.lower, R.lr, sp.pl, sp.pr);
+        RowVal tx, ty;
+        if (textured) {
+            tx = RowVal(E, tc[0].x, tc[1].x, tc[2].x);
+            ty = RowVal(E, tc[0].y, tc[1].y, tc[2].y);
+        }
         for (int x = xa; x < xb; x++, q.step()) {
             const int p = (y - ty0) * TW + (x - tx0);
             const float u = q.u();
@@ -2093,10 +2089,10 @@ __device__ uint64_t layer_walk(const JobDev &J, uint32_t t, const SubTri &st, in
             mask |= 1ull << p;
             bool op = flat_opaque;
             if (textured) {
-                const f2 tc = SS.t_left + SS.t_dir * u;
+                const f2 at = {tx.at(E.along(u)), ty.at(E.along(u))};
                 uint32_t no_count = 0;   // texel reads are counted where the survivors are shaded
-                op = tk == 1 ? (nearest(X, tc) >> 24) == 255
-                             : bilinear_channel(bilinear_taps(X, tc, no_count), 3) == 255;
+                op = tk == 1 ? (nearest(X, at) >> 24) == 255
+                             : bilinear_channel(bilinear_taps(X, at, no_count), 3) == 255;
             }
             opq |= (uint64_t)op << p;
         }
@@ -2120,29 +2116,42 @@ __device__ __forceinline__ void layer_chunk(const JobDev &J, const uint32_t *lis
                                             int px, int py, bool mine, int K, bool deferred, LayerPixel &P,
                                             uint32_t &frags, uint32_t &nans, uint32_t &oob)
 {
-    constexpr int TW = SW_LAYER_TW;
-    if (threadIdx.x < n) {
-        const uint32_t t = list[threadIdx.x];
+    constexpr int TW = SW_LAYER_TW, TH = SW_LAYER_TH;
+    // With few entries, 2, 4 or 8 lanes share an entry's rows: what a lane
+    // takes longest over are the replays from a large triangle's first row
+    // and from each span's first pixel.
+    const uint32_t sh = n <= 8 ? 3u : n <= 16 ? 2u : n <= 32 ? 1u : 0u;
+    const uint32_t e = threadIdx.x >> sh, part = threadIdx.x & ((1u << sh) - 1u);
+    if (threadIdx.x < n)
+        s_mask[threadIdx.x] = s_opq[threadIdx.x] = 0ull;
+    __syncthreads();
+    if (e < n) {
+        const uint32_t t = list[e];
         SubTri st[2];
         const int ns = tri_subs<true>(J, t, st);
-        LayerSub &L = s_sub[threadIdx.x];
-        uint64_t m = 0ull;
+        LayerSub &L = s_sub[e];
+        uint64_t m = 0ull, o = 0ull;
         if (ns == 1 && !st[0].v[0].clip && !st[0].v[1].clip && !st[0].v[2].clip) {
+            if (part == 0) {
 #pragma unroll
-            for (int k = 0; k < 3; k++) {
-                L.sx[k] = st[0].v[k].s.x;
-                L.sy[k] = st[0].v[k].s.y;
-                L.sz[k] = st[0].v[k].s.z;
-                L.a[k] = st[0].v[k].a;
+                for (int k = 0; k < 3; k++) {
+                    L.sx[k] = st[0].v[k].s.x;
+                    L.sy[k] = st[0].v[k].s.y;
+                    L.sz[k] = st[0].v[k].s.z;
+                    L.a[k] = st[0].v[k].a;
+                }
+                L.kind = st[0].front ? 3u : 1u;
             }
-            L.kind = st[0].front ? 3u : 1u;
-            m = layer_walk<GENERIC>(J, t, st[0], tx0, ty0, s_z + threadIdx.x * 64,
-                                    deferred ? s_opq + threadIdx.x : nullptr);
-        } else {
+            m = layer_walk<GENERIC>(J, t, st[0], tx0, ty0, (int)(part * (TH >> sh)), (int)((part + 1) * (TH >> sh)),
+                                    s_z + e * 64, deferred ? &o : nullptr);
+        } else if (part == 0) {
             L.kind = ns == 0 ? 0u : 4u;
             m = ns == 0 ? 0ull : ~0ull;   // near-clipped: every pixel lane sets it up itself
         }
-        s_mask[threadIdx.x] = m;
+        if (m)
+            atomicOr((unsigned long long *)&s_mask[e], (unsigned long long)m);
+        if (o)
+            atomicOr((unsigned long long *)&s_opq[e], (unsigned long long)o);
     }
     __syncthreads();
     const int x = tx0 + px, y = ty0 + py, p = py * TW + px;
@@ -2173,7 +2182,9 @@ __device__ __forceinline__ void layer_chunk(const JobDev &J, const uint32_t *lis
                     return 0u;
                 Interp q = sp.q;
                 q.steps(x - sp.x1);
-                return shade_from<GENERIC>(J, tt, S, R, sp, q.u(), oob);
+                Frag F;
+                frag_of(J, tt, S, R, sp, q.u(), F);
+                return shade_frag<GENERIC>(J, F, oob);
             });
         } else if (L.kind == 4u) {
             SubTri st[2];
@@ -2193,8 +2204,10 @@ __device__ __forceinline__ void layer_chunk(const JobDev &J, const uint32_t *lis
                 const float u = q.u();
                 layer_update(P, q.value(u), 2u * tt + (uint32_t)sub, K, deferred, frags, nans, [&] {
                     uint32_t no_count = 0;
-                    return deferred ? texture_from<GENERIC>(J, tt, S, R, sp, u, no_count)
-                                    : shade_from<GENERIC>(J, tt, S, R, sp, u, oob);
+                    Frag F;
+                    frag_of(J, tt, S, R, sp, u, F);
+                    return deferred ? frag_texture<GENERIC>(J, F, RowEnds(F.lower, F.lr, F.pl, F.pr), no_count)
+                                    : shade_frag<GENERIC>(J, F, oob);
                 });
             }
         }
@@ -2298,39 +2311,56 @@ __global__ __launch_bounds__(SW_LAYER_THREADS) void k_raster_layers(BatchDev B, 
                 }
                 __syncthreads();
             }
-        for (uint32_t c = 0; c < total; c += CH)
-            layer_chunk<GENERIC>(J, s_list + c, min(CH, total - c), s_sub, s_z, s_mask, s_opq, tx0, ty0, px, py, mine, K,
-                                 deferred, P, frags, nans, oob);
-    } else {
-        // too many for LDS: every triangle of the job in draw order, CH at a time
-        const int wave = (int)(threadIdx.x >> 6);
-        for (uint32_t base = 0; base < J.n_tris; base += CH) {
-            const uint32_t t = base + threadIdx.x;
+    }
+    // the tile's list, or, too long for LDS, every triangle of the job in draw
+    // order, CH at a time (one loop: layer_chunk's code is there once)
+    for (uint32_t pos = 0; pos < (listed ? total : J.n_tris); pos += CH) {
+        const uint32_t *list = s_list;
+        uint32_t n = 0;
+        if (listed) {
+            list += pos;
+            n = min(CH, total - pos);
+        } else {
+            const int wave = (int)(threadIdx.x >> 6);
+            const uint32_t t = pos + threadIdx.x;
             const bool cov = threadIdx.x < CH && t < J.n_tris && covers(t);
             const uint64_t bal = __ballot(cov);
             if (lane == 0)
                 s_wcount[wave] = (uint32_t)__popcll(bal);
             __syncthreads();
-            uint32_t before = 0, total = 0;
+            uint32_t before = 0;
             for (int k = 0; k < NT / 64; k++) {
                 before += k < wave ? s_wcount[k] : 0u;
-                total += s_wcount[k];
+                n += s_wcount[k];
             }
             if (cov)
                 s_list[before + (uint32_t)__popcll(bal & lt_mask)] = t;
             __syncthreads();
-            layer_chunk<GENERIC>(J, s_list, total, s_sub, s_z, s_mask, s_opq, tx0, ty0, px, py, mine, K, deferred, P,
-                                 frags, nans, oob);
         }
+        layer_chunk<GENERIC>(J, list, n, s_sub, s_z, s_mask, s_opq, tx0, ty0, px, py, mine, K, deferred, P, frags, nans,
+                             oob);
     }
     if (mine && deferred) {
         // shade the base and the surviving layers (sequences in the slots)
         const int x = tx0 + px, y = ty0 + py;
-        P.bc = P.bseq != 0xFFFFFFFFu ? shade_pixel<GENERIC>(J, P.bseq, x, y, oob) : 0u;
+        // (one copy of the shading's code for the base, k = K, and the layers)
+        for (int k = K; k >= 0; k--) {
+            uint32_t seq = P.bseq;
+            bool used = P.bseq != 0xFFFFFFFFu;
 #pragma unroll
-        for (int k = 0; k < KMAX; k++)
-            if (k < K)
-                P.lc[k] = P.lz[k] != maxz ? shade_pixel<GENERIC>(J, P.lc[k], x, y, oob) : 0u;
+            for (int m = 0; m < KMAX; m++)
+                if (m == k && m < K) {
+                    seq = P.lc[m];
+                    used = P.lz[m] != maxz;
+                }
+            const uint32_t color = used ? shade_pixel<GENERIC>(J, seq, x, y, oob) : 0u;
+            if (k == K)
+                P.bc = color;
+#pragma unroll
+            for (int m = 0; m < KMAX; m++)
+                if (m == k && m < K)
+                    P.lc[m] = color;
+        }
     }
     if (mine) {
         const int x = tx0 + px, y = ty0 + py;

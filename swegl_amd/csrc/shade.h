@@ -118,6 +118,8 @@ struct TexView {
 };
 SW_D uint32_t texel(const TexView &X, int64_t i) { return X.p ? ro(X.p)[i] : X.one; }
 
+struct Texel2 { uint32_t x, y; };   // two neighbours, aligned as one
+
 // The four texels and weights of one bilinear sample.
 struct BilTaps {
     uint32_t p[4];
@@ -151,14 +153,22 @@ SW_D BilTaps bilinear_taps(const TexView &X, f2 t, uint32_t &oob)
         // both taps of either axis inside the bitmap, and products of 30
         // bits at most: 24-bit multiplies and 32-bit indices
         const uint32_t r1 = __umul24((uint32_t)v1m, (uint32_t)tw), r2 = __umul24((uint32_t)v2m, (uint32_t)tw);
-        const uint32_t i0 = r1 + (uint32_t)u1m, i1 = r2 + (uint32_t)u1m, i2 = r1 + (uint32_t)u2m,
-                       i3 = r2 + (uint32_t)u2m;
         T.p[0] = T.p[1] = T.p[2] = T.p[3] = X.one;
         if (X.p) {
-            T.p[0] = ro(X.p)[i0];
-            T.p[1] = ro(X.p)[i1];
-            T.p[2] = ro(X.p)[i2];
-            T.p[3] = ro(X.p)[i3];
+            // the taps of a row are neighbours unless the second wraps
+            const uint32_t i0 = r1 + (uint32_t)u1m, i1 = r2 + (uint32_t)u1m;
+            if (u2m) {
+                const Texel2 a = *(const SW_RO Texel2 *)(ro(X.p) + i0), b = *(const SW_RO Texel2 *)(ro(X.p) + i1);
+                T.p[0] = a.x;
+                T.p[2] = a.y;
+                T.p[1] = b.x;
+                T.p[3] = b.y;
+            } else {
+                T.p[0] = ro(X.p)[i0];
+                T.p[1] = ro(X.p)[i1];
+                T.p[2] = ro(X.p)[r1];
+                T.p[3] = ro(X.p)[r2];
+            }
         }
     } else {
         const int64_t lim = (int64_t)tw * th;
@@ -267,79 +277,33 @@ SW_D uint32_t combine(uint32_t color, int32_t light_i)
     return out;
 }
 
-// Shader state of one triangle half and one scanline
-// (prepare_for_triangle / _upper / _lower / _scanline, pixel_shaders.cpp:88-158
-// and :304-346).
-struct TriAttr {
-    f3 w[3];    // v_world of the y-sorted vertices
-    f3 n[3];    // normal_world, negated when the triangle is inverted
-    f2 t[3];    // tex_coords * (width, height)
-};
-
-struct ScanShade {
-    f3 v, vdir, n, ndir;
-    f2 t_left, t_dir;
-};
-
-SW_D ScanShade prepare_scanline(const TriAttr &A, bool lower, bool lr, float pl, float pr)
-{
-    f3 vleft, vright, vld, vrd, nleft, nright, nld, nrd;
-    f2 sst, sstd;
-    const f2 sltd = A.t[2] - A.t[0];
-    if (!lower) {
-        vleft = A.w[0];
-        vright = A.w[0];
-        nleft = A.n[0];
-        nright = A.n[0];
-        if (lr) {
-            vld = A.w[1] - A.w[0];
-            vrd = A.w[2] - A.w[0];
-            nld = A.n[1] - A.n[0];
-            nrd = A.n[2] - A.n[0];
-        } else {
-            vld = A.w[2] - A.w[0];
-            vrd = A.w[1] - A.w[0];
-            nld = A.n[2] - A.n[0];
-            nrd = A.n[1] - A.n[0];
-        }
-        sst = A.t[0];
-        sstd = A.t[1] - A.t[0];
-    } else {
-        if (lr) {
-            vright = A.w[0];
-            vrd = A.w[2] - A.w[0];
-            vleft = A.w[1];
-            vld = A.w[2] - A.w[1];
-            nright = A.n[0];
-            nrd = A.n[2] - A.n[0];
-            nleft = A.n[1];
-            nld = A.n[2] - A.n[1];
-        } else {
-            vleft = A.w[0];
-            vld = A.w[2] - A.w[0];
-            vright = A.w[1];
-            vrd = A.w[2] - A.w[1];
-            nleft = A.n[0];
-            nld = A.n[2] - A.n[0];
-            nright = A.n[1];
-            nrd = A.n[2] - A.n[1];
-        }
-        sst = A.t[1];
-        sstd = A.t[2] - A.t[1];
+// One quantity over a scanline (prepare_for_triangle / _upper / _lower /
+// _scanline, pixel_shaders.cpp:88-158 and :304-346): a0, a1, a2 at the
+// y-sorted vertices.  The long side runs from vertex 0 to 2, the short one
+// from 0 to 1 in the upper half and 1 to 2 in the lower; the left end lies on
+// the short side when the long one is on the right (lr).  The reference's
+// left + (right - left) * u is `base` + `d` * (lr ? -u : u) here: d is the
+// short end minus the long one, and negation is exact.
+struct RowEnds {
+    bool lower, lr;
+    float ps, pL;   // progresses along the short and the long side
+    SW_D RowEnds(bool lower_, bool lr_, float pl, float pr)
+        : lower(lower_), lr(lr_), ps(lr_ ? pl : pr), pL(lr_ ? pr : pl)
+    {
     }
-    ScanShade S;
-    S.v = vleft + vld * pl;
-    S.vdir = vright + vrd * pr - S.v;
-    S.n = nleft + nld * pl;
-    S.ndir = nright + nrd * pr - S.n;
-    if (lr) {
-        S.t_left = sst + sstd * pl;
-        S.t_dir = A.t[0] + sltd * pr - S.t_left;
-    } else {
-        S.t_left = A.t[0] + sltd * pl;
-        S.t_dir = sst + sstd * pr - S.t_left;
+    SW_D float along(float u) const { return lr ? -u : u; }
+};
+struct RowVal {
+    float base, d;
+    SW_D RowVal() {}
+    SW_D RowVal(const RowEnds &E, float a0, float a1, float a2)
+    {
+        const float s0 = E.lower ? a1 : a0, s1 = E.lower ? a2 : a1;
+        const float s = s0 + (s1 - s0) * E.ps, l = a0 + (a2 - a0) * E.pL;
+        base = E.lr ? s : l;
+        d = s - l;
     }
-    return S;
-}
+    SW_D float at(float su) const { return base + d * su; }
+};
 
 }  // namespace sw
