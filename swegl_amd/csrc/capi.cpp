@@ -1124,7 +1124,7 @@ static void wave_tile(const swegl_ctx *c, const std::vector<JobIn> &jobs, int &t
 }
 
 // Per-viewport scratch of one job: frustum coordinates, marks, tile
-// rectangles, the big list, and with DoF the pre-DoF colour and code bytes,
+// rectangles, the big list, and with DoF the pre-DoF colours and alphas,
 // with layers the flattened layer colour.
 struct JobScratch {
     float4 *ndc = nullptr;
@@ -1142,7 +1142,7 @@ static size_t job_scratch_sizes(const swegl_scene *s, const swegl_viewport_desc 
     sz[1] = V;
     sz[2] = T * 8;
     sz[3] = T * 4;
-    sz[4] = v.post_shader != SWEGL_POST_NULL ? P * 5 : 0;   // colour, then one code byte per pixel
+    sz[4] = v.post_shader != SWEGL_POST_NULL ? P * 5 : 0;   // colour, then one alpha byte per pixel
     sz[5] = v.transparency_layer_count > 0 ? P * 4 : 0;
     return sz[0] + sz[1] + sz[2] + sz[3] + sz[4] + sz[5];
 }
@@ -1231,10 +1231,10 @@ static int build_wave(swegl_ctx *c, Lane &L, const std::vector<JobIn> &jobs, Wav
         J.V.cam = f3{v.camera_position[0], v.camera_position[1], v.camera_position[2]};
         J.surface = v.color->buf.as<uint32_t>();
         J.surface_pitch = v.color->w;
-        J.dofc = nullptr;
+        J.dofa = nullptr;
         if (dof) {
             J.out_color = vs.dof;
-            J.dofc = (uint8_t *)vs.dof + (size_t)v.w * v.h * 4;
+            J.dofa = (uint8_t *)vs.dof + (size_t)v.w * v.h * 4;
             J.out_pitch = v.w;
             J.out_ox = v.x;
             J.out_oy = v.y;

@@ -99,6 +99,12 @@ SW_D float sqrt_rn(float x)
     return __builtin_fmaf(__builtin_fmaf(-g, g, x), h, g);
 }
 
+// floor(x / c) of a tap count 1 <= c <= 1024 and a sum x <= 255 c of 8-bit
+// channels, from rc, v_rcp_f32 of c: (x + 1/2) / c lies at least 1 / 2c =
+// 4.8e-4 from a whole number, and the error of rc, 1 ulp, and the rounding
+// move a value below 256 by less than 5e-5.
+SW_D uint32_t tap_mean(uint32_t x, float rc) { return (uint32_t)__builtin_fmaf((float)x, rc, 0.5f * rc); }
+
 // Several quotients over one denominator, in div_rn's range.
 struct FDiv {
     float b, r;

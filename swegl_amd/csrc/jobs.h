@@ -51,9 +51,10 @@ struct NodeDev {
 // Bin limit of layered waves: on 8x8 tiles a smaller limit would send most
 // triangles of a close-up mesh to the big list, which every tile scans.
 #define SW_LAYER_BIG_TILES 32
-// Depth-of-field output tile (pixels) of one 256-thread workgroup.
+// Depth-of-field output tile (pixels) of one workgroup of SW_DOF_NT threads.
 #define SW_DOF_TW 64
-#define SW_DOF_TH 16
+#define SW_DOF_TH 32
+#define SW_DOF_NT 512
 __host__ __device__ inline uint32_t dof_blocks(int w, int h)
 {
     return (uint32_t)(((w + SW_DOF_TW - 1) / SW_DOF_TW) * ((h + SW_DOF_TH - 1) / SW_DOF_TH));
@@ -86,7 +87,7 @@ struct JobDev {
     uint32_t *tid;            // optional winning draw sequence, w*h
     int32_t shader;           // SWEGL_SHADER_*
     int32_t post;             // SWEGL_POST_*
-    uint8_t *dofc;            // DoF: per pixel (blur factor != 0) | radius << 1, w*h
+    uint8_t *dofa;            // DoF: alpha per pixel, w*h (out_color then holds b, g, r and dof_code)
     int32_t layers;           // transparency layers (0: none)
     uint32_t *tflat;          // with layers: flattened layer colour per pixel, w*h
     float fdist, fdepth;

@@ -813,11 +813,11 @@ __device__ __forceinline__ float blur_factor(float z, float fdist, float fdepth,
 
 // What the depth-of-field pass reads of a pixel: whether its blur factor is
 // nonzero, and its radius in the bits above.
-__device__ __forceinline__ uint8_t dof_code(float z, float fdist, float fdepth, int rmax, const FDiv &by, bool fast)
+__device__ __forceinline__ uint32_t dof_code(float z, float fdist, float fdepth, int rmax, const FDiv &by, bool fast)
 {
     const float bf = blur_factor(z, fdist, fdepth, (float)rmax, by, fast);
     const int radius = min(max(cvtt(bf), 0), rmax);   // bf is in [0, rmax] for finite inputs
-    return (uint8_t)((bf != 0.0f ? 1 : 0) | (radius << 1));
+    return (bf != 0.0f ? 1u : 0u) | (uint32_t)radius << 1;
 }
 
 // ------------------------------------------------------------- k_raster
@@ -1701,7 +1701,11 @@ __device__ __forceinline__ uint32_t raster_tile(const BatchDev &B, const JobDev 
                 if (have)
                     color = shade_frag<GENERIC>(K, F, oob);
             }
-            K.out_color[(int64_t)(y - K.out_oy) * K.out_pitch + (x - K.out_ox)] = color;
+            // with depth of field the colour waits for its code below
+            if (K.dofa)
+                keys[i] = (uint64_t)__float_as_uint(z) << 32 | color;
+            else
+                K.out_color[(int64_t)(y - K.out_oy) * K.out_pitch + (x - K.out_ox)] = color;
             const int64_t zo = (int64_t)(y - K.V.vy) * K.V.vw + (x - K.V.vx);
             K.zbuf[zo] = z;
             if (K.tid)
@@ -1709,19 +1713,23 @@ __device__ __forceinline__ uint32_t raster_tile(const BatchDev &B, const JobDev 
         }
         id = id_next;
     }
-    // The depth-of-field pass reads this code instead of z.  A loop of its
-    // own keeps its registers out of the shading loop's peak.
+    // What the depth-of-field pass reads: b, g, r with dof_code above them,
+    // and alpha in a plane of its own.  A loop of its own keeps its registers
+    // out of the shading loop's peak.
     const JobDev &D = reread(jobs, jidx);
-    if (D.dofc) {
+    if (D.dofa) {
         const FDiv dof_by(D.fdepth - 1.0f);
         const bool dof_fast = D.fdepth - 1.0f >= 1.0f && D.fdepth - 1.0f <= 0x1p20f;
         for (int i = threadIdx.x; i < npix; i += NT) {
             const int x = tr.x0 + (i % TW), y = tr.y0 + (i / TW);
             if (x >= tr.x1 || y >= tr.y1)
                 continue;
-            const float z = __uint_as_float((uint32_t)(keys[i] >> 32));   // max_z where empty
-            D.dofc[(int64_t)(y - D.V.vy) * D.V.vw + (x - D.V.vx)] =
-                dof_code(z, D.fdist, D.fdepth, D.rmax, dof_by, dof_fast);
+            const unsigned long long k = keys[i];   // this thread's, written above
+            const uint32_t color = (uint32_t)k;
+            const uint32_t code =
+                dof_code(__uint_as_float((uint32_t)(k >> 32)), D.fdist, D.fdepth, D.rmax, dof_by, dof_fast);
+            D.out_color[(int64_t)(y - D.out_oy) * D.out_pitch + (x - D.out_ox)] = (color & 0xFFFFFFu) | code << 24;
+            D.dofa[(int64_t)(y - D.V.vy) * D.V.vw + (x - D.V.vx)] = (uint8_t)(color >> 24);
         }
     }
     if (B.stats) {
@@ -1743,8 +1751,8 @@ __device__ __forceinline__ void fill_empty(const BatchDev &B, const JobDev *__re
     const JobDev &J = jobs[find_job<JTILE>(B, jobs, g)];
     const int lt = (int)(g - J.tile_base), tx = lt % J.tiles_x, ty = lt / J.tiles_x;
     const float maxz = __uint_as_float(SW_MAX_Z_BITS);
-    uint8_t code = 0;
-    if (J.dofc) {
+    uint32_t code = 0;
+    if (J.dofa) {
         const FDiv by(J.fdepth - 1.0f);
         const bool fast = J.fdepth - 1.0f >= 1.0f && J.fdepth - 1.0f <= 0x1p20f;
         code = dof_code(maxz, J.fdist, J.fdepth, J.rmax, by, fast);
@@ -1753,13 +1761,13 @@ __device__ __forceinline__ void fill_empty(const BatchDev &B, const JobDev *__re
         const int x = tx * TW + i % TW, y = ty * TH + i / TW;   // viewport-relative
         if (x >= J.V.vw || y >= J.V.vh)
             continue;
-        J.out_color[(int64_t)(y + J.V.vy - J.out_oy) * J.out_pitch + (x + J.V.vx - J.out_ox)] = 0u;
+        J.out_color[(int64_t)(y + J.V.vy - J.out_oy) * J.out_pitch + (x + J.V.vx - J.out_ox)] = code << 24;
         const int64_t zo = (int64_t)y * J.V.vw + x;
         J.zbuf[zo] = maxz;
         if (J.tid)
             J.tid[zo] = 0xFFFFFFFFu;
-        if (J.dofc)
-            J.dofc[zo] = code;
+        if (J.dofa)
+            J.dofa[zo] = 0;
     }
 }
 
@@ -2419,152 +2427,189 @@ __global__ __launch_bounds__(256) void k_tcopy(BatchDev B, uint32_t job, const J
 
 // ---------------------------------------------------------------- k_dof
 // Depth of field (build spec of post_shader_depth_box, post_shaders.hpp:51-131
-// with remap_clipped, lerp.hpp:24-43): 64x16 output pixels per block, colour
-// and blur factor of the tile plus an R_max halo staged in LDS.
-// Exact floor(x / c) for 1 <= c <= 1024 and x < 2^18 (a tap count and a
-// sum of 8-bit channels) as a high multiply by m = ceil(2^32 / c): the
-// error x * (m * c - 2^32) / 2^32 < 2^18 * 2^10 / 2^32 stays below 1/c.
-struct DofRecip {
-    uint32_t m[4 * SW_MAX_DOF_RADIUS * SW_MAX_DOF_RADIUS + 1];
-};
-constexpr DofRecip make_dof_recip()
-{
-    DofRecip t{};
-    for (uint32_t c = 2; c <= 4u * SW_MAX_DOF_RADIUS * SW_MAX_DOF_RADIUS; c++)
-        t.m[c] = 0xFFFFFFFFu / c + 1u;
-    return t;
-}
-__constant__ DofRecip k_dof_recip = make_dof_recip();
-__device__ __forceinline__ uint32_t div_count(uint32_t x, uint32_t c)
-{
-    return c == 1 ? x : __umulhi(x, k_dof_recip.m[c]);
-}
-
+// with remap_clipped, lerp.hpp:24-43): 64x32 output pixels per block, colour
+// and blur factor of the tile plus a halo staged in LDS.
 // LDS bytes of a k_dof<RMAX> workgroup: two tap words per cell of the
-// output tile plus an RMAX halo on every side (20 KB for RMAX 8: eight
-// workgroups on a CU).
+// output tile plus an RMAX halo on every side (30 KB for RMAX 8).
 __host__ __device__ inline size_t dof_lds_bytes(int RMAX)
 {
     return (size_t)(SW_DOF_TW + 2 * RMAX) * (SW_DOF_TH + 2 * RMAX) * 8;
 }
 
-// 256 threads as 64 columns x 4 rows.  Consecutive workgroups run on
-// different XCDs (round robin over 8), so the job's tiles are dealt out in
-// 8 contiguous runs, one per XCD: neighbouring tiles, whose halos overlap,
-// then share that XCD's L2.  The raster stored, per pixel, whether its blur
-// factor is nonzero (an "unfocused" tap) and its clamped radius.
-// RMAX bounds the wave's halo (the loads below are unrolled for it): the
-// launch picks 8 when no job of the launch has a larger radius.
+// SW_DOF_NT threads as 64 columns x 8 rows.  Bound by the instructions a
+// pixel and by one round of loads: at 3840x2160 with radii to 16 it takes
+// 29 us (75 MB, 14 us of copy), 68 before; at 1920x1080 with radii to 8 10 us,
+// 15 before; eight views 24, 39 before; a 1280x720 box 16, 22 before.  What
+// it gained from: a row a wave (58 to 37 us at 3840x2160; a window dealt out
+// cell by cell costs a division a cell), means from one reciprocal rather than
+// a gathered table (37 to 29), one word a pixel, the taller tile.  A halo as
+// wide as the tile's own largest radius was no faster: the radii are read
+// before the halo then.
+// Consecutive workgroups run on different XCDs (round robin over 8), so the
+// job's tiles are dealt out in 8 contiguous runs, one per XCD: neighbouring
+// tiles, whose halos overlap, then share that XCD's L2.  The raster left b, g, r and
+// dof_code in one word a pixel -- whether it is an "unfocused" tap, and its
+// clamped radius -- and alpha apart, which only copied pixels need.
+// RMAX bounds the job's halo (the loads below are unrolled for it, and the
+// LDS window has its pitch): the launch picks 8 when no job of the launch
+// has a larger radius.  The halo's cells are much of the work, so the tile is
+// 64x32 (1.9 cells a pixel at radius 8, 3.0 at 16; 64x16: 2.5 and 4.5, and 26
+// us against 24 for the eight views, 38 against 29 at 3840x2160).  64x64 on
+// 1,024 threads gains at radius 16 (26) and costs at 8.
+// The window is loaded a row of the tile a wave, so that a row's address and
+// its bounds are scalar: the tile's own rows, which the output needs in any
+// case, the rows above and below it, and the columns beside it, several rows
+// a wave.
 // Each LDS cell holds a tap as two words, (b, r) and (g, 1) as 16-bit
 // halves for an unfocused pixel, zeros for a focused pixel or a cell
 // outside the viewport (never an unfocused tap, which is what the
 // reference's clipped loops give): a tap is one 64-bit LDS read and two
 // adds, its count coming with the colour.
+// The box's (2r)^2 taps come from exclusive prefix sums along the rows of
+// the window, two reads a row (a row's sums stay below 2^16: at most 96 cells
+// of 255), from SW_DOF_PREFIX on, where two reads a row beat six taps (the
+// 1280x720 box of radius 5: 22.7 to 19.3 us when this went in).
+#define SW_DOF_PREFIX 3
 template <int RMAX>
-__global__ __launch_bounds__(256) void k_dof(BatchDev B, const JobDev *__restrict__ jobs)
+__global__ __launch_bounds__(SW_DOF_NT) void k_dof(BatchDev B, const JobDev *__restrict__ jobs)
 {
-    extern __shared__ uint2 s_dyn[];
+    extern __shared__ uint2 s_tap[];
+    constexpr int TW = SW_DOF_TW, TH = SW_DOF_TH, ROWS = SW_DOF_NT / TW, PER = TH / ROWS, P = TW + 2 * RMAX;
+    static_assert(TW == 64 && TH % ROWS == 0 && 64 % (2 * RMAX) == 0, "a wave loads whole rows");
     const JobDev &J = jobs[find_job<JD>(B, jobs, blockIdx.x)];
     const uint32_t n = dof_blocks(J.V.vw, J.V.vh), q = n / 8;
     uint32_t lb = blockIdx.x - J.dblock0;
     if (lb < 8 * q)
         lb = (lb % 8) * q + lb / 8;
-    const int bx = (J.V.vw + SW_DOF_TW - 1) / SW_DOF_TW;
-    const int ox = (int)(lb % bx) * SW_DOF_TW, oy = (int)(lb / bx) * SW_DOF_TH;   // viewport-relative
-    const int R = J.rmax;
-    const int SW = SW_DOF_TW + 2 * R, SH = SW_DOF_TH + 2 * R;
-    // The LDS window has the pitch of the largest halo (P) and SH rows; its
-    // cells are dealt to the threads in order, NC / 256 each (the window of
-    // the largest halo is a multiple of 256 cells), so no lane idles on a
-    // ragged row.
-    constexpr int P = SW_DOF_TW + 2 * RMAX, NC = P * (SW_DOF_TH + 2 * RMAX), PERT = NC / 256;
-    static_assert(NC % 256 == 0, "the LDS window is dealt out in whole rounds of 256 cells");
-    uint2 *s_tap = s_dyn;
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    // Every load of the halo is issued before the first is used, so the
-    // workgroup waits for memory once rather than once per row.  A cell
-    // outside the viewport (or past the window's SW columns) loads the
-    // tile's first pixel instead (no branch per cell) and is zeroed after.
-    // Offsets are 32-bit: a surface holds at most 2^30 words.
-    const SW_RO uint32_t *colr = ro(J.out_color);
-    const SW_RO uint8_t *code = ro(J.dofc);
-    const int cbase = (J.V.vy - J.out_oy) * J.out_pitch + (J.V.vx - J.out_ox);   // colour of viewport (0, 0)
-    const int safe_c = cbase + oy * J.out_pitch + ox, safe_k = oy * J.V.vw + ox;
-    uint32_t cv[PERT], kv[PERT];
-    bool okv[PERT];
-#pragma unroll
-    for (int k = 0; k < PERT; k++) {
-        const int i = (int)threadIdx.x + 256 * k, r = i / P, c = i % P;
-        const int ly = oy - R + r, lx = ox - R + c;
-        okv[k] = r < SH && c < SW && ly >= 0 && ly < J.V.vh && lx >= 0 && lx < J.V.vw;
-        cv[k] = colr[okv[k] ? cbase + ly * J.out_pitch + lx : safe_c];   // the raster's output: read-only here
-        kv[k] = code[okv[k] ? ly * J.V.vw + lx : safe_k];
-    }
-    // the output pixels' own colours and codes (in the rows just loaded:
-    // cache hits)
-    constexpr int PER = SW_DOF_TH / 4;
-    uint32_t src[PER], own[PER];
+    const int bx = (J.V.vw + TW - 1) / TW;
+    const int ox = (int)(lb % bx) * TW, oy = (int)(lb / bx) * TH;   // viewport-relative
+    const int R = J.rmax, vw = J.V.vw, vh = J.V.vh, pitch = J.out_pitch;
+    const int tx = threadIdx.x & 63, ty = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // Offsets are 32-bit: a surface holds at most 2^30 words.  A cell outside
+    // the viewport loads one inside and is zeroed after (no branch per cell);
+    // every load is issued before the first is used.
+    const SW_RO uint32_t *colr = ro(J.out_color) + ((J.V.vy - J.out_oy) * pitch + (J.V.vx - J.out_ox));
+    const SW_RO uint8_t *alpha = ro(J.dofa);
+    const int x = ox + tx, xin = min(x, vw - 1);
+    uint32_t own[PER], al[PER];
 #pragma unroll
     for (int j = 0; j < PER; j++) {
-        const int x = ox + tx, y = oy + ty + 4 * j;
-        const bool in = x < J.V.vw && y < J.V.vh;
-        src[j] = colr[in ? cbase + y * J.out_pitch + x : safe_c];
-        own[j] = code[in ? y * J.V.vw + x : safe_k];
+        const int y = min(oy + ty + ROWS * j, vh - 1);
+        own[j] = colr[y * pitch + xin];
+        al[j] = alpha[y * vw + xin];
+    }
+    // the rows above and below: row h of 2R is -R + h, past the tile from R on
+    constexpr int NV = (2 * RMAX + ROWS - 1) / ROWS;
+    uint32_t vert[NV];
+#pragma unroll
+    for (int k = 0; k < NV; k++) {
+        const int h = ty + ROWS * k, y = oy + (h < R ? h - R : h - R + TH);
+        vert[k] = 0;
+        if (h < 2 * R && y >= 0 && y < vh)   // the same in every lane
+            vert[k] = colr[y * pitch + xin];
+    }
+    // the columns beside: SIDE lanes a row, RMAX on either side
+    constexpr int SIDE = 2 * RMAX, SROWS = 64 / SIDE, NS = (TH + 2 * RMAX + ROWS * SROWS - 1) / (ROWS * SROWS);
+    const int e = tx % SIDE, scol = e < RMAX ? e - RMAX : e - RMAX + TW;   // tile-relative
+    const int sx = ox + scol, sxin = min(max(sx, 0), vw - 1);
+    const bool sok = sx >= 0 && sx < vw;
+    uint32_t side[NS];
+#pragma unroll
+    for (int k = 0; k < NS; k++) {
+        const int y = oy - R + (ty + ROWS * k) * SROWS + tx / SIDE;
+        side[k] = colr[min(max(y, 0), vh - 1) * pitch + sxin];
+        if (!sok || y < 0 || y >= vh)
+            side[k] = 0;
+    }
+    auto put = [&](int row, int col, uint32_t v) {   // tile-relative cell
+        const uint32_t w = v & 1u << 24 ? v : 0u;     // bit 24: unfocused
+        s_tap[(row + RMAX) * P + col + RMAX] = make_uint2(w & 0x00FF00FFu, w >> 8 & 0x000100FFu);
+    };
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const int row = ty + ROWS * j;
+        put(row, tx, x < vw && oy + row < vh ? own[j] : 0u);
     }
 #pragma unroll
-    for (int k = 0; k < PERT; k++) {
-        const uint32_t w = okv[k] && (kv[k] & 1u) ? ((cv[k] & 0x00FFFFFFu) | (1u << 24)) : 0u;
-        s_tap[threadIdx.x + 256 * k] = make_uint2(w & 0x00FF00FFu, (w >> 8) & 0x00FF00FFu);
+    for (int k = 0; k < NV; k++) {
+        const int h = ty + ROWS * k;
+        if (h < 2 * R)
+            put(h < R ? h - R : h - R + TH, tx, x < vw ? vert[k] : 0u);
+    }
+#pragma unroll
+    for (int k = 0; k < NS; k++) {
+        const int h = (ty + ROWS * k) * SROWS + tx / SIDE;
+        if (h < TH + 2 * R)
+            put(h - R, scol, side[k]);
     }
     __syncthreads();
+    const bool prefix = J.post == 1 && R >= SW_DOF_PREFIX;
+    if (prefix) {
+        // exclusive prefix sums along each row, one wave a row, 64 cells at a time
+        for (int r = ty; r < TH + 2 * R; r += ROWS) {
+            uint2 carry = make_uint2(0, 0);
+            for (int c0 = 0; c0 < P; c0 += 64) {
+                const int i = (r + RMAX - R) * P + c0 + tx;
+                const bool in = c0 + tx < P;
+                const uint2 v = in ? s_tap[i] : make_uint2(0, 0);
+                const uint2 t = make_uint2(carry.x + wave_incl_scan(v.x), carry.y + wave_incl_scan(v.y));
+                if (in)
+                    s_tap[i] = make_uint2(t.x - v.x, t.y - v.y);
+                carry = make_uint2(__shfl(t.x, 63), __shfl(t.y, 63));
+            }
+        }
+        __syncthreads();
+    }
+    if (x >= vw)
+        return;
 #pragma unroll
     for (int j = 0; j < PER; j++) {
-        const int py = ty + 4 * j, px = tx;
-        const int x = ox + px, y = oy + py;
-        if (x >= J.V.vw || y >= J.V.vh)
-            continue;
-        const int c = (py + R) * P + (px + R);
-        const int radius = (int)(own[j] >> 1);
-        uint32_t out = src[j];
+        const int py = ty + ROWS * j, y = oy + py;
+        if (y >= vh)
+            break;
+        const int c = (py + RMAX) * P + tx + RMAX;
+        const int radius = (int)(own[j] >> 25);
+        uint32_t out = (own[j] & 0xFFFFFFu) | al[j] << 24;
         if (radius != 0) {
-            // With radius <= 8 a sum has at most 256 taps of 255, under 2^16:
-            // blue and red add as the halves of one word, green and the
-            // count as the halves of another.
-            constexpr bool PACKED = RMAX <= 8;
+            // Blue and red add as the halves of one word, green and the count
+            // as the halves of another: nine taps of 255, or the 256 of a box
+            // of radius 8, stay below 2^16.  A larger box adds them apart.
             uint32_t br = 0, gc = 0, b = 0, g = 0, r = 0, count = 0;
-            auto tap = [&](int k) {   // LDS cell k
-                const uint2 w = s_tap[k];
-                if (PACKED) {
-                    br += w.x;
-                    gc += w.y;
-                } else {
-                    b += w.x & 0xFFFFu;
-                    r += w.x >> 16;
-                    g += w.y & 0xFFFFu;
-                    count += w.y >> 16;
-                }
+            auto add = [&](uint2 w) {
+                br += w.x;
+                gc += w.y;
             };
-            if (J.post == 1) {   // box [x-r, x+r) x [y-r, y+r)
+            auto unpack = [&] {
+                b += br & 0xFFFFu;
+                r += br >> 16;
+                g += gc & 0xFFFFu;
+                count += gc >> 16;
+                br = gc = 0;
+            };
+            if (prefix) {   // box, [x-r, x+r) x [y-r, y+r)
+                for (int a = -radius; a < radius; a++) {
+                    const uint2 lo = s_tap[c + a * P - radius], hi = s_tap[c + a * P + radius];
+                    add(make_uint2(hi.x - lo.x, hi.y - lo.y));
+                    if (RMAX > 8)
+                        unpack();
+                }
+            } else if (J.post == 1) {
                 for (int a = -radius; a < radius; a++)
-                    for (int e = -radius; e < radius; e++)
-                        tap(c + a * P + e);
+                    for (int f = -radius; f < radius; f++)
+                        add(s_tap[c + a * P + f]);
             } else {             // 3x3 taps at {-r, 0, r}
                 const int dr = radius * P;
 #pragma unroll
                 for (int a = -1; a <= 1; a++)
 #pragma unroll
-                    for (int e = -1; e <= 1; e++)
-                        tap(c + a * dr + e * radius);
+                    for (int f = -1; f <= 1; f++)
+                        add(s_tap[c + a * dr + f * radius]);
             }
-            if (PACKED) {
-                b = br & 0xFFFFu;
-                r = br >> 16;
-                g = gc & 0xFFFFu;
-                count = gc >> 16;
+            unpack();
+            if (count) {
+                const float rc = __builtin_amdgcn_rcpf((float)count);
+                out = tap_mean(b, rc) | tap_mean(g, rc) << 8 | tap_mean(r, rc) << 16 | 255u << 24;
             }
-            if (count)
-                out = (uint32_t)(uint8_t)div_count(b, count) | ((uint32_t)(uint8_t)div_count(g, count) << 8) |
-                      ((uint32_t)(uint8_t)div_count(r, count) << 16) | (255u << 24);
         }
         J.surface[(int64_t)(y + J.V.vy) * J.surface_pitch + (x + J.V.vx)] = out;
     }
@@ -2676,9 +2721,9 @@ hipError_t launch_dof(const BatchDev &B, uint32_t blocks, int max_radius, hipStr
     if (!blocks)
         return hipSuccess;
     if (max_radius <= 8)
-        LAUNCH_CHECK(k_dof<8>, dim3(blocks), dim3(256), dof_lds_bytes(8), s, B, B.jobs);
+        LAUNCH_CHECK(k_dof<8>, dim3(blocks), dim3(SW_DOF_NT), dof_lds_bytes(8), s, B, B.jobs);
     else
-        LAUNCH_CHECK(k_dof<SW_MAX_DOF_RADIUS>, dim3(blocks), dim3(256), dof_lds_bytes(SW_MAX_DOF_RADIUS), s, B,
+        LAUNCH_CHECK(k_dof<SW_MAX_DOF_RADIUS>, dim3(blocks), dim3(SW_DOF_NT), dof_lds_bytes(SW_MAX_DOF_RADIUS), s, B,
                      B.jobs);
     return hipSuccess;
 }

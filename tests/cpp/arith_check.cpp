@@ -48,9 +48,20 @@ __global__ void quotients(uint32_t count, unsigned long long *bad)
         atomicAdd(&bad[2], d);
 }
 
+__global__ void means(unsigned long long *bad)
+{
+    const uint32_t c = blockIdx.x + 1;
+    const float rc = __builtin_amdgcn_rcpf((float)c);
+    unsigned long long d = 0;
+    for (uint32_t x = threadIdx.x; x <= 255u * c; x += 256u)
+        d += sw::tap_mean(x, rc) != x / c;
+    if (d)
+        atomicAdd(&bad[3], d);
+}
+
 int main()
 {
-    unsigned long long *bad = nullptr, h[3] = {1, 1, 1};
+    unsigned long long *bad = nullptr, h[4] = {1, 1, 1, 1};
     if (hipMalloc((void **)&bad, sizeof h) != hipSuccess || hipMemset(bad, 0, sizeof h) != hipSuccess) {
         std::printf("no device\n");
         return 2;
@@ -59,10 +70,12 @@ int main()
     for (uint32_t part = 0; part < 4; part++)
         unary<<<4096, 256>>>(lo + part * (n / 4), n / 4 + (part == 3), bad);
     quotients<<<count / 256, 256>>>(count, bad);
+    means<<<1024, 256>>>(bad);
     if (hipMemcpy(h, bad, sizeof h, hipMemcpyDeviceToHost) != hipSuccess) {
         std::printf("device error\n");
         return 2;
     }
-    std::printf("mismatches: reciprocal %llu, square root %llu, quotient %llu\n", h[0], h[1], h[2]);
-    return h[0] || h[1] || h[2] ? 1 : 0;
+    std::printf("mismatches: reciprocal %llu, square root %llu, quotient %llu, mean %llu\n", h[0], h[1], h[2],
+                h[3]);
+    return h[0] || h[1] || h[2] || h[3] ? 1 : 0;
 }
