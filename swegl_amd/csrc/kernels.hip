@@ -575,8 +575,8 @@ __device__ void order_tiles(const BatchDev &B, uint32_t queue)
 }
 
 // ------------------------------------------------------------- k_front
-// Tiles of more than 256 entries: the most pixels that one lane replays on its
-// own; smallest chunk (pixels) of a listed triangle.
+// Tiles whose lanes take a triangle each (raster_tile): the most pixels that
+// one lane replays on its own; smallest chunk (pixels) of a listed triangle.
 #define SW_LANE_PIXELS 96
 #define SW_CHUNK_PIXELS 8
 // Per triangle, in one pass: the visibility marks (renderer.cpp:83-185: a
@@ -931,9 +931,10 @@ __device__ __forceinline__ void walk_rows(const Setup &S, int wy0, int wy1, RowF
 }
 
 // Any triangle: near-clipped (two sub-triangles), non-finite, of any size.
+// Its fragments in rows [wy0, wy1) and columns [wx0, wx1) of the tile.
 __device__ void raster_depth_any(const JobDev &J, uint32_t t, uint32_t i0, uint32_t i1, uint32_t i2, TileRect tr,
-                                 int wy0, int wy1, unsigned long long *keys, int TW, uint32_t &frags,
-                                 uint32_t &nans, unsigned long long *slots, int nslot)
+                                 int wy0, int wy1, int wx0, int wx1, unsigned long long *keys, int TW,
+                                 uint32_t &frags, uint32_t &nans, unsigned long long *slots, int nslot)
 {
     SubTri st[2];
     int ns = tri_subs_v<true>(J, i0, i1, i2, st);
@@ -948,7 +949,7 @@ __device__ void raster_depth_any(const JobDev &J, uint32_t t, uint32_t i0, uint3
             Span sp;
             if (!span_of(R, J.V, sp))
                 return;
-            int xa = max(sp.x1, tr.x0), xb = min(sp.x2, tr.x1);
+            int xa = max(sp.x1, wx0), xb = min(sp.x2, wx1);
             if (xa >= xb)
                 return;
             Interp q = sp.q;
@@ -1073,11 +1074,12 @@ __device__ __forceinline__ void side_steps(PSide &s, int n)
 }
 
 // The fragments of plain triangle t (vertices i0, i1, i2) in rows [wy0, wy1)
-// of the tile.
+// and columns [wx0, wx1) of the tile.
 template <int TW, bool SLOTS>
 __device__ __forceinline__ void plain_depth(const TileView &W, const PTri &T, uint32_t t, uint32_t i0, uint32_t i1,
-                                            uint32_t i2, int wy0, int wy1, unsigned long long *keys,
-                                            unsigned long long *slots, int nslot, uint32_t &frags, uint32_t &nans)
+                                            uint32_t i2, int wy0, int wy1, int wx0, int wx1,
+                                            unsigned long long *keys, unsigned long long *slots, int nslot,
+                                            uint32_t &frags, uint32_t &nans)
 {
     const PVert a = T.a, b = T.b, c = T.c;
     // fill_triangle's facing (cross_z_sign, whose product is zero or at least
@@ -1145,7 +1147,7 @@ __device__ __forceinline__ void plain_depth(const TileView &W, const PTri &T, ui
         // span_of: the row's columns, then its sides' progresses and depths
         const float lx = lr ? S.x : L.x, rx = lr ? L.x : S.x;
         const int x1 = max((int)ceilf(lx), W.vx);
-        const int xa = max(x1, W.tr.x0), xb = min((int)ceilf(rx), W.tr.x1);
+        const int xa = max(x1, wx0), xb = min((int)ceilf(rx), wx1);
         if (xa < xb) {
             const float uL = div_rn(L.ta, L.ba, rcp_rn(L.ba)), uS = div_rn(S.ta, S.ba, rcp_rn(S.ba));
             const float zL = L.v0 + L.v1 * uL, zS = S.v0 + S.v1 * uS;
@@ -1432,10 +1434,10 @@ __device__ __forceinline__ uint32_t raster_tile(const BatchDev &B, const JobDev 
 
     uint32_t frags = 0, nans = 0, oob = 0;
     // Replay the tile's binned triangles, then the job's big triangles whose
-    // rectangle touches this tile.  Up to NT of them are cut into chunks of
-    // rows, of about an equal number of pixels (from the screen bounding
-    // boxes) and about as many as there are lanes, so that a few large
-    // triangles occupy every lane.  With more, a lane takes a
+    // rectangle touches this tile.  Up to NT / 2 of them are cut into chunks of
+    // rows, or of parts of a row's columns, of about an equal number of pixels
+    // (from the screen bounding boxes) and about as many as there are lanes, so
+    // that a few large triangles occupy every lane.  With more, a lane takes a
     // triangle of its own, all rows, if it is plain and not one that covers
     // more than SW_LANE_PIXELS pixels of the tile, on which its lane would
     // spend several times what the others do; those are listed and cut up
@@ -1443,7 +1445,10 @@ __device__ __forceinline__ uint32_t raster_tile(const BatchDev &B, const JobDev 
     // in this phase with 20-40 lanes busy, and one lane per triangle a tile
     // of 330 entries with one large among them 65 us.  The 640x480 cube's
     // raster 45 -> 31 us, the 800x600 demo scene's 78 -> 47; chunks of at
-    // least 16 or 32 pixels: 34 and 40 us for the cube.)
+    // least 16 or 32 pixels: 34 and 40 us for the cube.  Parts of rows took
+    // the cube from 28 to 24 us, where two triangles a tile kept 32 of 256
+    // lanes busy with a row of 32 pixels each; lists of up to NT / 2 rather
+    // than NT the demo scene from 42 to 36, of NT / 4 no further.)
     __shared__ uint32_t s_tri[NT], s_rows[NT], s_first[NT], s_wsum[NT / 64], s_n;
     // The tile's entries: placed by k_front in its job's fixed layout
     // (every triangle whose rectangle holds the tile; marks are checked
@@ -1520,7 +1525,7 @@ __device__ __forceinline__ uint32_t raster_tile(const BatchDev &B, const JobDev 
         return (tx >= (int)(r.x & 0xFFFF)) & (tx <= (int)(r.y & 0xFFFF)) & (ty >= (int)(r.x >> 16)) &
                (ty <= (int)(r.y >> 16));
     };
-    const bool many = entries > NT;
+    const bool many = entries > NT / 2;
     uint32_t listed = entries;
     if (many) {
         if (threadIdx.x == 0)
@@ -1560,7 +1565,8 @@ __device__ __forceinline__ uint32_t raster_tile(const BatchDev &B, const JobDev 
                         ((k & flags & SW_BIN_LARGE) && rows_of(T, true, ry0, ry1) > SW_LANE_PIXELS))
                         list(t);
                     else
-                        plain_depth<TW, SLOTS>(W, T, t, i0, i1, i2, W.tr.y0, W.tr.y1, keys, slots, NSLOT, frags, nans);
+                        plain_depth<TW, SLOTS>(W, T, t, i0, i1, i2, W.tr.y0, W.tr.y1, W.tr.x0, W.tr.x1, keys, slots, NSLOT,
+                                               frags, nans);
                 }
                 if (e + NT >= nb)
                     break;
@@ -1588,6 +1594,7 @@ __device__ __forceinline__ uint32_t raster_tile(const BatchDev &B, const JobDev 
     for (uint32_t base = 0; base < last; base += NT) {
         uint32_t t = 0, area = 0;
         int ry0 = tr.y0, ry1 = tr.y0;
+        bool plain = false;
         if (base + threadIdx.x < last) {
             uint32_t i0, i1, i2;
             bool check = false, large = true, have = true;
@@ -1597,7 +1604,7 @@ __device__ __forceinline__ uint32_t raster_tile(const BatchDev &B, const JobDev 
             else
                 have = entry(base + threadIdx.x, t, check, large);
             if (have && load(t, check, i0, i1, i2, T)) {   // unmarked: no chunks
-                const bool plain = is_plain(T);
+                plain = is_plain(T);
                 area = (uint32_t)rows_of(T, plain, ry0, ry1);
                 if (again && base + threadIdx.x < nb && plain && !(large && area > SW_LANE_PIXELS))
                     area = 0;   // done above
@@ -1616,14 +1623,21 @@ __device__ __forceinline__ uint32_t raster_tile(const BatchDev &B, const JobDev 
         __syncthreads();
         const uint32_t per = max(block_total() / (uint32_t)NT, (uint32_t)SW_CHUNK_PIXELS);
         const uint32_t rows = (uint32_t)(ry1 - ry0);
-        const uint32_t nch = area ? min(max(area / per, 1u), rows) : 0u;
+        // whole rows a chunk, or 2^cols parts of one
+        uint32_t nch = area ? max((uint32_t)((float)area * __builtin_amdgcn_rcpf((float)per)), 1u) : 0u, cols = 0;
+        if (nch > rows) {
+            while (cols < 3 && rows << (cols + 1) <= nch)
+                cols++;
+            nch = rows << cols;
+        }
         __syncthreads();   // s_wsum read, s_tri too
         // exclusive prefix of the chunk counts over the block
         const uint32_t incl = wave_incl_scan(nch);
         if (lane == 63)
             s_wsum[wave] = incl;
         s_tri[threadIdx.x] = t;
-        s_rows[threadIdx.x] = (uint32_t)(ry0 - tr.y0) | ((uint32_t)(ry1 - tr.y0) << 8) | (nch << 16);
+        s_rows[threadIdx.x] = (uint32_t)(ry0 - tr.y0) | ((uint32_t)(ry1 - tr.y0) << 8) | (nch << 16) |
+                             cols << 28 | (plain ? 1u << 31 : 0u);
         __syncthreads();
         uint32_t before = 0;
         for (int k = 0; k < wave; k++)
@@ -1643,17 +1657,20 @@ __device__ __forceinline__ uint32_t raster_tile(const BatchDev &B, const JobDev 
             }
             // s_first is non-decreasing and i < total, so entry lo has a chunk holding i
             // (an entry without chunks shares its s_first with the next entry)
-            const uint32_t pk = s_rows[lo], n = pk >> 16, ch = i - s_first[lo];
+            const uint32_t pk = s_rows[lo], lc = pk >> 28 & 7u, n = (pk >> 16 & 0xFFFu) >> lc, part = i - s_first[lo];
+            const uint32_t ch = part >> lc, col = part & ((1u << lc) - 1u);
             const int r0 = tr.y0 + (int)(pk & 0xFF), nr = (int)((pk >> 8) & 0xFF) - (int)(pk & 0xFF);
-            const int wy0 = r0 + (int)((uint32_t)nr * ch / n), wy1 = r0 + (int)((uint32_t)nr * (ch + 1) / n);
+            const float rn = __builtin_amdgcn_rcpf((float)n);   // tap_mean: nr, ch and n are at most 64
+            const int wy0 = r0 + (int)tap_mean((uint32_t)nr * ch, rn), wy1 = r0 + (int)tap_mean((uint32_t)nr * (ch + 1), rn);
+            const int wx0 = tr.x0 + (int)(col * TW >> lc), wx1 = min(tr.x0 + (int)((col + 1u) * TW >> lc), tr.x1);
             const uint32_t tt = s_tri[lo];
             uint32_t i0, i1, i2;
             PTri T;
             load(tt, false, i0, i1, i2, T);
-            if (is_plain(T))
-                plain_depth<TW, SLOTS>(W, T, tt, i0, i1, i2, wy0, wy1, keys, slots, NSLOT, frags, nans);
+            if (pk >> 31)
+                plain_depth<TW, SLOTS>(W, T, tt, i0, i1, i2, wy0, wy1, wx0, wx1, keys, slots, NSLOT, frags, nans);
             else
-                raster_depth_any(reread(jobs, jidx), tt, i0, i1, i2, tr, wy0, wy1, keys, TW, frags, nans,
+                raster_depth_any(reread(jobs, jidx), tt, i0, i1, i2, tr, wy0, wy1, wx0, wx1, keys, TW, frags, nans,
                                  SLOTS ? slots : nullptr, NSLOT);
         }
         __syncthreads();   // the LDS tables are rewritten by the next NT
@@ -2439,7 +2456,7 @@ __host__ __device__ inline size_t dof_lds_bytes(int RMAX)
 // SW_DOF_NT threads as 64 columns x 8 rows.  Bound by the instructions a
 // pixel and by one round of loads: at 3840x2160 with radii to 16 it takes
 // 29 us (75 MB, 14 us of copy), 68 before; at 1920x1080 with radii to 8 10 us,
-// 15 before; eight views 24, 39 before; a 1280x720 box 16, 22 before.  What
+// 15 before; four such views 24, 39 before; a 1231x717 box 16, 22 before.  What
 // it gained from: a row a wave (58 to 37 us at 3840x2160; a window dealt out
 // cell by cell costs a division a cell), means from one reciprocal rather than
 // a gathered table (37 to 29), one word a pixel, the taller tile.  A halo as
@@ -2454,7 +2471,7 @@ __host__ __device__ inline size_t dof_lds_bytes(int RMAX)
 // LDS window has its pitch): the launch picks 8 when no job of the launch
 // has a larger radius.  The halo's cells are much of the work, so the tile is
 // 64x32 (1.9 cells a pixel at radius 8, 3.0 at 16; 64x16: 2.5 and 4.5, and 26
-// us against 24 for the eight views, 38 against 29 at 3840x2160).  64x64 on
+// us against 24 for four views, 38 against 29 at 3840x2160).  64x64 on
 // 1,024 threads gains at radius 16 (26) and costs at 8.
 // The window is loaded a row of the tile a wave, so that a row's address and
 // its bounds are scalar: the tile's own rows, which the output needs in any
@@ -2468,7 +2485,7 @@ __host__ __device__ inline size_t dof_lds_bytes(int RMAX)
 // The box's (2r)^2 taps come from exclusive prefix sums along the rows of
 // the window, two reads a row (a row's sums stay below 2^16: at most 96 cells
 // of 255), from SW_DOF_PREFIX on, where two reads a row beat six taps (the
-// 1280x720 box of radius 5: 22.7 to 19.3 us when this went in).
+// 1231x717 box of radius 5: 22.7 to 19.3 us when this went in).
 #define SW_DOF_PREFIX 3
 template <int RMAX>
 __global__ __launch_bounds__(SW_DOF_NT) void k_dof(BatchDev B, const JobDev *__restrict__ jobs)

@@ -105,6 +105,26 @@ def test_crowded_tiles_among_empty_ones(ctx, tile, w, h):
         ctx.set_raster_groups(4)
 
 
+@pytest.mark.parametrize("tile", [(16, 16), (32, 32), (64, 32), (64, 64)])
+@pytest.mark.parametrize("n", [1, 2, 5, 64, 65, 128, 129, 256, 257])
+def test_few_large_triangles(ctx, n, tile):
+    """Tiles of a few triangles, whose rows are cut into parts, and of as many
+    as are listed at most, and one more; some are near-clipped."""
+    rng = np.random.default_rng(n)
+    s = flat_scene(triangles(rng, n, 1.2, z=(-1.0, 2.2)).tolist(), double_sided=True)
+    vps = [view(150, 110)]
+    want = oracle.render(s, vps)[0]
+    ctx.set_tile_auto(False)
+    ctx.set_tile(*tile)
+    try:
+        got = gpu_render(ctx, s, vps)[0]
+        compare(got, want)
+        assert got.stats["fragments"] == want.stats["fragments"]
+    finally:
+        ctx.set_tile_auto(True)
+        ctx.set_tile(32, 32)
+
+
 def test_texture_coordinates_not_finite(ctx):
     rng = np.random.default_rng(5)
     s = flat_scene(triangles(rng, 40, 0.4).tolist(), double_sided=True)
