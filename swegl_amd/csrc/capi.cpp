@@ -1285,8 +1285,7 @@ static int build_wave(swegl_ctx *c, Lane &L, const std::vector<JobIn> &jobs, Wav
     // the job's per-tile share of 1.25 entries per triangle, at least 512 (a
     // batch mixes scenes of very different densities, and a crowded tile --
     // a horizon, a stack of meshes -- holds 8-19 times its job's share); a
-    // job whose busiest tile needs more takes the filled layout, the others
-    // keep theirs
+    // tile with more takes the filled layout, the others keep theirs
     W.fixed = false;
     W.fixed_total = 0;
     if ((!arena || L.own_views) && !W.layers && W.tiles && tris_total < 0x40000000ull) {   // (SW_BIN_CHECK, SW_BIN_LARGE: top bits)

@@ -114,17 +114,19 @@ struct WorldArgs {
 // Tile counters: tile g's bin count at tile_count[g * SW_TILE_PAD] and its
 // fill rank (entries placed so far) one word later, a 128-byte line per tile, so the binning
 // atomics of different tiles spread over all memory channels instead of
-// queueing on the few that a dense array maps to.  Words 4 to 7 of line i hold
+// queueing on the few that a dense array maps to.  Word 2 of line i names the
+// i-th tile that passed its fixed layout (BatchDev::fixed); words 4 to 7 hold
 // slots 4i to 4i + 3 of the raster's claim order (item_slot), written by
 // k_bin_fill's first blocks.
 #define SW_TILE_PAD 32
+#define SW_NO_OFFSET 0xFFFFFFFFu   // (bins hold fewer entries)
 
 struct BatchDev {
     const JobDev *jobs;
     uint32_t n_jobs;
     uint32_t n_tiles;         // total tiles over all jobs
     uint32_t *tile_count;     // [n_tiles * SW_TILE_PAD], see SW_TILE_PAD
-    uint32_t *tile_offset;    // [n_tiles + 1]
+    uint32_t *tile_offset;    // [n_tiles + 1]: a tile's first entry in bins, or SW_NO_OFFSET
     uint32_t *tile_cursor;    // tile_count + 1: the fill ranks
     uint32_t *bins;           // [capacity]: the counted, scanned and filled layout
     uint32_t *bins_fixed;     // the fixed layout's entries (JobDev::bin_base, tile_cap)
@@ -133,10 +135,11 @@ struct BatchDev {
     uint32_t *ctr;            // counter words, layout below
     uint32_t stats;           // 1: accumulate the statistics counters
     // 1: k_front places every entry in its job's fixed layout as it counts
-    // it (marks unchecked); only a job with a tile holding more entries than
-    // its tile_cap (its word at SW_CTR_BIG0 + n_jobs + job set, and
-    // SW_CTR_OVERFLOW) is filled by k_bin_fill into the counted layout,
-    // after the offsets scan; 0: the counted layout for every job
+    // it (marks unchecked); a tile with more entries than its job's tile_cap
+    // is listed (word 2 of counter line i names the i-th, SW_CTR_OVERFLOW
+    // counts them; its job's word at SW_CTR_BIG0 + n_jobs + job is set) and
+    // filled by k_bin_fill into the counted layout, at the offset k_front's
+    // last block gives it; 0: the counted layout for every tile
     uint32_t fixed;
     uint32_t order;           // 1: k_bin_fill writes the claim order (0: layered waves, which have none)
     uint32_t split;           // a tile of more entries is SW_BANDS items; 0xFFFFFFFF: none is
@@ -166,7 +169,7 @@ struct BatchDev {
 // index k mod SW_TICKET_GROUPS, then one of the finished groups, each on
 // its own 128-byte line (same-address atomics serialise where they execute)
 #define SW_TICKET_GROUPS 32
-#define SW_CTR_OVERFLOW (SW_CTR_TOTAL + 32)   // nonzero: a tile passed tile_cap
+#define SW_CTR_OVERFLOW (SW_CTR_TOTAL + 32)   // tiles that passed tile_cap
 // Each raster queue's number of items, then of empty tiles after them; the
 // claims of those (a line of its own for each queue)
 #define SW_CTR_ITEMS (SW_CTR_TOTAL + 34)

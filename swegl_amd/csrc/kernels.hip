@@ -137,13 +137,15 @@ __global__ __launch_bounds__(256) void k_world(WorldArgs W)
 // world_to_camera_or_frustum (vertex_shaders.hpp:35-52, 61-71) per viewport:
 // frustum coordinates and cleared visibility marks.
 // It also zeroes the tile counts and fill ranks and the counter words
-// [w0, w0 + n_words) that the binning kernels after it accumulate into.
+// [w0, w0 + n_words) that the binning kernels after it accumulate into, and
+// marks every tile as without an offset.
 __global__ __launch_bounds__(256) void k_vertex(BatchDev B, uint32_t w0, uint32_t n_words, const JobDev *__restrict__ jobs)
 {
     const uint32_t gi = blockIdx.x * 256u + threadIdx.x, stride = gridDim.x * 256u;
     for (uint32_t k = gi; k < B.n_tiles; k += stride) {
         B.tile_count[k * SW_TILE_PAD] = 0;
         B.tile_cursor[k * SW_TILE_PAD] = 0;
+        B.tile_offset[k] = SW_NO_OFFSET;
     }
     for (uint32_t k = gi; k < n_words; k += stride)
         B.ctr[w0 + k] = 0;
@@ -590,8 +592,17 @@ __device__ void order_tiles(const BatchDev &B, uint32_t queue)
 // rectangle is counted here; k_bin_fill, which runs after all marks are
 // set, places only triangles whose three vertices are marked, and the
 // raster checks the marks of big-list triangles.  The last block to finish
-// scans the tile counts into the bin offsets (the claim order is written by
-// k_bin_fill's last block, off this kernel's critical path).
+// gives the tiles that k_bin_fill will fill their bin offsets (the claim order
+// is written by k_bin_fill's first blocks, off this kernel's critical path).
+// With the fixed layout those are the tiles that passed their capacity, listed
+// by the one entry that found each full; the others keep their entries where
+// they are.  (Scanning every tile's count for the sake of a few took one
+// workgroup 18 us for 8,160 tiles, placing every triangle of such a job again
+// 10 to 15, and noting the overflow with two read-modify-writes a wave 23 on
+// four 1920x1080 views of 500,000 stacked triangles: k_front + k_bin_fill 85 +
+// 35 us, 45 + 24 now; the 999,698-triangle field at 3840x2160 51 + 25 and 33 +
+// 13.  64 times a tile's share instead of 16 gained as much, at 240 MB a
+// buffer set and 0.1 ms of a first frame.)
 __global__ __launch_bounds__(256) void k_front(BatchDev B, const JobDev *__restrict__ jobs)
 {
     const int jidx = find_job<JT>(B, jobs, blockIdx.x);
@@ -640,7 +651,6 @@ __global__ __launch_bounds__(256) void k_front(BatchDev B, const JobDev *__restr
     }
     // one aggregated atomic per distinct tile per wave and round; with a
     // tile capacity the count's old value places the entry
-    bool overflow = false;
     for (int k = 0; __any(k < ntiles); k++) {
         const bool act = k < ntiles;
         uint32_t key = 0;
@@ -654,14 +664,18 @@ __global__ __launch_bounds__(256) void k_front(BatchDev B, const JobDev *__restr
             if (act && rank < J.tile_cap)
                 B.bins_fixed[J.bin_base + (size_t)(key - J.tile_base) * J.tile_cap + rank] =
                     t | (self_marked ? 0u : SW_BIN_CHECK) | (large ? SW_BIN_LARGE : 0u);
-            overflow |= act && rank >= J.tile_cap;
+            if (act && rank == J.tile_cap) {
+                // one entry of a tile finds it full: the tile is listed for
+                // the filled layout and its job noted (seen by other XCDs)
+                const uint32_t i = atomicAdd(B.ctr + SW_CTR_OVERFLOW, 1u);
+                __hip_atomic_store(&B.tile_count[(size_t)i * SW_TILE_PAD + 2], key, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(B.ctr + SW_CTR_BIG0 + B.n_jobs + jidx, 1u, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+            }
         } else {
             wave_add<false>(B.tile_count, key * SW_TILE_PAD, act);
         }
-    }
-    if (__any(overflow) && __lane_id() == 0) {   // every lane of a block has the block's job
-        atomicOr(B.ctr + SW_CTR_BIG0 + B.n_jobs + jidx, 1u);
-        atomicOr(B.ctr + SW_CTR_OVERFLOW, 1u);
     }
     // The last block to finish scans.  The counts are device-scope atomics,
     // performed at the memory side, not in an XCD's L2: each wave waits
@@ -687,9 +701,24 @@ __global__ __launch_bounds__(256) void k_front(BatchDev B, const JobDev *__restr
     __syncthreads();
     if (!s_last)
         return;
-    // the offsets serve the filled layout only
-    if (!B.fixed || __hip_atomic_load(B.ctr + SW_CTR_OVERFLOW, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+    // the offsets serve the filled layout only: of every tile, or of the full
+    // ones listed above
+    if (!B.fixed) {
         scan_offsets<256>(B);
+        return;
+    }
+    const uint32_t full = __hip_atomic_load(B.ctr + SW_CTR_OVERFLOW, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __shared__ uint32_t s_next;
+    if (threadIdx.x == 0)
+        s_next = 0;
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < full; i += 256u) {
+        const uint32_t g = __hip_atomic_load(&B.tile_count[(size_t)i * SW_TILE_PAD + 2], __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT);
+        const uint32_t n = __hip_atomic_load(&B.tile_count[(size_t)g * SW_TILE_PAD], __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT);
+        B.tile_offset[g] = atomicAdd(&s_next, n);
+    }
 }
 
 // ----------------------------------------------------------- k_bin_fill
@@ -704,8 +733,8 @@ __global__ __launch_bounds__(256) void k_bin_fill(BatchDev B, const JobDev *__re
             order_tiles<256>(B, blockIdx.x);
         return;
     }
-    // k_front placed every entry of a job unless one of its tiles
-    // overflowed: then only the statistics, if asked for, are counted here
+    // k_front placed every entry of a job unless one of its tiles was full;
+    // otherwise only the statistics, if asked for, are counted here
     const uint32_t blk = blockIdx.x - SW_RASTER_QUEUES;
     const int jidx = find_job<JT>(B, jobs, blk);
     const bool place = !B.fixed || B.ctr[SW_CTR_BIG0 + B.n_jobs + jidx] != 0;
@@ -755,12 +784,18 @@ __global__ __launch_bounds__(256) void k_bin_fill(BatchDev B, const JobDev *__re
             key = J.tile_base + (ty0 + ky) * J.tiles_x + (tx0 + kx);
             entries++;
         }
-        // the entry's place: the tile's offset (read while the rank's atomic is
-        // in flight) plus its rank among the tile's entries so far
-        const uint32_t off = act ? ro(B.tile_offset)[key] : 0u;
-        const uint32_t rank = wave_add<true>(B.tile_cursor, key * SW_TILE_PAD, act);
+        // the entry's place: the tile's offset plus its rank among the tile's
+        // entries so far; tiles whose fixed layout holds them have no offset
+        // (their counts would tell as well, but lie on the lines the ranks'
+        // atomics work on: 45 us instead of 24 for four views of stacked
+        // triangles)
+        const uint32_t off = act ? ro(B.tile_offset)[key] : SW_NO_OFFSET;
+        const bool put = off != SW_NO_OFFSET;
+        if (!__any(put))
+            continue;
+        const uint32_t rank = wave_add<true>(B.tile_cursor, key * SW_TILE_PAD, put);
         const uint32_t pos = off + rank;
-        if (act && pos < B.bin_capacity)
+        if (put && pos < B.bin_capacity)
             B.bins[pos] = t;
     }
     if (!B.stats)
@@ -1452,14 +1487,15 @@ __device__ __forceinline__ uint32_t raster_tile(const BatchDev &B, const JobDev 
     __shared__ uint32_t s_tri[NT], s_rows[NT], s_first[NT], s_wsum[NT / 64], s_n;
     // The tile's entries: placed by k_front in its job's fixed layout
     // (every triangle whose rectangle holds the tile; marks are checked
-    // here), or, when a tile of the job passed its capacity, by k_bin_fill
-    // at the scanned offset (marked triangles only; the count also held
-    // unmarked ones); then the job's big list.
-    const bool fixed = B.fixed != 0 && B.ctr[SW_CTR_BIG0 + B.n_jobs + jidx] == 0;
+    // here), or, when they passed its capacity, by k_bin_fill at the offset
+    // found for the tile (marked triangles only; the count also held unmarked
+    // ones); then the job's big list.
+    const uint32_t counted = B.tile_count[g * SW_TILE_PAD];
+    const bool fixed = B.fixed != 0 && counted <= J.tile_cap;
     uint32_t nb;
     const uint32_t *bins;
     if (fixed) {
-        nb = min(B.tile_count[g * SW_TILE_PAD], J.tile_cap);
+        nb = counted;
         bins = B.bins_fixed + J.bin_base + (size_t)lt * J.tile_cap;
     } else {
         nb = B.tile_cursor[g * SW_TILE_PAD];

@@ -143,3 +143,32 @@ def test_one_job_overflows_its_tiles(ctx, graph):
         compare(got[k][0], oracle.render(s, v)[0], colour_tol=1)
     if not graph:
         assert st["fragments"] > 0
+
+
+@pytest.mark.parametrize("order", [(0, 1), (1, 0)])
+@pytest.mark.parametrize("crowd", [500, 700, 6000])
+def test_full_tiles_among_others(ctx, crowd, order):
+    """Tiles of one job hold more than the fixed bin layout has room for,
+    beside tiles that do not and a job without any; half of the triangles face
+    away.  Eager, again with the same buffers, and replayed."""
+    from test_oracle_scene import flat_scene, view
+    rng = np.random.default_rng(crowd)
+
+    def spots(n, spread):
+        c = np.concatenate([rng.uniform(-spread, spread, (n, 1, 2)), rng.uniform(-1, 0.5, (n, 1, 1))], -1)
+        return c + rng.uniform(-0.03, 0.03, (n, 3, 3)) * [1, 1, 0.3]
+
+    pairs = [(flat_scene(np.concatenate([spots(crowd, 0.05), spots(900, 0.8)]).tolist()), [view(403, 301)]),
+             (flat_scene(spots(300, 0.6).tolist()), [view(190, 170)])]
+    pairs = [pairs[k] for k in order]
+    want = [oracle.render(s, vps)[0] for s, vps in pairs]
+    batch = Batch(ctx, pairs)
+    for graph in (False, False, True, True):
+        st = batch.render(graph=graph)
+        for got, w in zip(batch.frames(), want):
+            compare(got[0], w)
+        for k in ("fragments", "drawn_subtriangles"):
+            assert st[k] == sum(w.stats[k] for w in want)
+    batch.render(stats=False)
+    for got, w in zip(batch.frames(), want):
+        compare(got[0], w)
