@@ -1387,9 +1387,11 @@ static int carve_resources(Arena &A, std::vector<Wave> &waves, ResPtr &out)
 // `untimed`: no profiling events (capture, and the allocation-free path).
 // The front-end stages go on `fs` (the lane's stream when null); with
 // another stream, `fdone` is recorded there after them and the lane's
-// stream waits for it before the raster.
+// stream waits for it before the raster.  `with_table`: the job table, of
+// one job, goes along with the first kernel's arguments; otherwise it is
+// already at R.jobs.
 static int launch_wave(swegl_ctx *c, Lane &L, const ResPtr &R, const Wave &W, bool first_wave, bool untimed,
-                       bool want_stats, hipStream_t fs = nullptr, hipEvent_t fdone = nullptr)
+                       bool want_stats, bool with_table, hipStream_t fs = nullptr, hipEvent_t fdone = nullptr)
 {
     const bool capturing = untimed;
     BatchDev B;
@@ -1422,7 +1424,7 @@ static int launch_wave(swegl_ctx *c, Lane &L, const ResPtr &R, const Wave &W, bo
     } while (0)
     if (!fs)
         fs = st;
-    STAGE("vertex", fs, launch_vertex(B, W.vblk, zero0, W.n_ctr - zero0, fs));
+    STAGE("vertex", fs, launch_vertex(B, W.vblk, zero0, W.n_ctr - zero0, with_table ? W.jd.data() : nullptr, fs));
     STAGE("front", fs, launch_front(B, W.tblk, fs));
     // with two streams, the fill's own completion records fdone (no
     // separate marker on fstream, which would hold up the next front end)
@@ -1566,6 +1568,13 @@ static int render_jobs(swegl_ctx *c, Lane &L, const std::vector<JobIn> &all, swe
             // everything on the context stream when other work was queued
             // there since the last pipelined render
             hipStream_t fs = c->fstream;
+            // One job's table goes along with the first kernel, except where
+            // a front end of more blocks than CUs would then start together
+            // with the raster before it and take its workgroups' places: the
+            // 999,698-triangle 1920x1080 field 96 us a frame with the copy
+            // ahead of it, 114 without; the 800x600 demo scene 57 and 53.
+            const bool one = waves[0].jd.size() == 1 &&
+                             (c->pipe_seq != c->op_seq || waves[0].tblk <= (uint32_t)std::max(1, c->n_cus));
             if (c->pipe_seq != c->op_seq) {
                 HIPCHK(hipEventRecord(c->tail, c->stream));
                 HIPCHK(hipStreamWaitEvent(fs, c->tail, 0));
@@ -1576,8 +1585,8 @@ static int render_jobs(swegl_ctx *c, Lane &L, const std::vector<JobIn> &all, swe
             c->pipe_seq = c->op_seq - 1;   // until this render is fully queued
             const size_t jb = waves[0].jd.size() * sizeof(JobDev);
             if (c->f_recorded[p])
-                HIPCHK(hipEventSynchronize(c->f_done[p]));   // the slot's last copy has ended
-            if (c->job_pinned_n[p] < jb) {
+                HIPCHK(hipEventSynchronize(c->f_done[p]));   // the slot's last front end has ended
+            if (!one && c->job_pinned_n[p] < jb) {
                 if (c->job_pinned[p])
                     (void)hipHostFree(c->job_pinned[p]);
                 c->job_pinned[p] = nullptr;
@@ -1585,12 +1594,14 @@ static int render_jobs(swegl_ctx *c, Lane &L, const std::vector<JobIn> &all, swe
                 HIPCHK(hipHostMalloc(&c->job_pinned[p], std::max<size_t>(jb, 4096), hipHostMallocDefault));
                 c->job_pinned_n[p] = std::max<size_t>(jb, 4096);
             }
-            memcpy(c->job_pinned[p], waves[0].jd.data(), jb);
+            hipError_t ce = hipSuccess;
             c->f_recorded[p] = true;
-            hipError_t ce = hipMemcpyAsync(R.jobs + waves[0].job_offset, c->job_pinned[p], jb,
-                                           hipMemcpyHostToDevice, fs);
+            if (!one) {
+                memcpy(c->job_pinned[p], waves[0].jd.data(), jb);
+                ce = hipMemcpyAsync(R.jobs + waves[0].job_offset, c->job_pinned[p], jb, hipMemcpyHostToDevice, fs);
+            }
             if ((rc = ce != hipSuccess ? fail(SWEGL_EIO, "job table copy: %s", hipGetErrorString(ce)) : 0) ||
-                (rc = launch_wave(c, L, R, waves[0], true, false, stats != nullptr, fs, c->f_done[p]))) {
+                (rc = launch_wave(c, L, R, waves[0], true, false, stats != nullptr, one, fs, c->f_done[p]))) {
                 // whatever reached fstream is waited for by the context stream
                 (void)hipEventRecord(c->f_done[p], fs);
                 (void)hipStreamWaitEvent(c->stream, c->f_done[p], 0);
@@ -1604,9 +1615,10 @@ static int render_jobs(swegl_ctx *c, Lane &L, const std::vector<JobIn> &all, swe
         c->op_seq++;   // serial: the next pipelined render waits for it
     }
     for (size_t w = 0; w < waves.size(); w++) {
-        if ((rc = upload(L, R.jobs + waves[w].job_offset, waves[w].jd.data(),
-                         waves[w].jd.size() * sizeof(JobDev))) ||
-            (rc = launch_wave(c, L, R, waves[w], w == 0, false, stats != nullptr)))
+        const bool one = waves[w].jd.size() == 1;
+        if ((!one && (rc = upload(L, R.jobs + waves[w].job_offset, waves[w].jd.data(),
+                                  waves[w].jd.size() * sizeof(JobDev)))) ||
+            (rc = launch_wave(c, L, R, waves[w], w == 0, false, stats != nullptr, one)))
             return rc;
     }
     return stats ? read_stats(c, L, R.ctr, stats) : SWEGL_OK;
@@ -1650,7 +1662,7 @@ static int render_jobs_noalloc(swegl_ctx *c, const std::vector<JobIn> &all, sweg
     HIPCHK(hipEventRecord(c->noalloc_done, c->stream));
     c->noalloc_used = true;
     for (size_t w = 0; w < waves.size(); w++)
-        if ((rc = launch_wave(c, c->lane0, R, waves[w], w == 0, true, stats != nullptr)))
+        if ((rc = launch_wave(c, c->lane0, R, waves[w], w == 0, true, stats != nullptr, false)))
             return rc;
     return stats ? read_stats(c, c->lane0, R.ctr, stats) : SWEGL_OK;
 }
@@ -1732,7 +1744,7 @@ static int render_jobs_graph(swegl_ctx *c, const std::vector<JobIn> &all, swegl_
         int lrc = SWEGL_OK;
         const ResPtr GR = res_ptr(g->res);
         for (size_t w = 0; lrc == SWEGL_OK && w < waves.size(); w++)
-            lrc = launch_wave(c, c->lane0, GR, waves[w], w == 0, true, stats != nullptr);
+            lrc = launch_wave(c, c->lane0, GR, waves[w], w == 0, true, stats != nullptr, false);
         hipGraph_t graph = nullptr;
         hipError_t ee = hipStreamEndCapture(c->stream, &graph);
         g->graph = graph;   // destroyed with the entry if anything below fails

@@ -139,7 +139,7 @@ __global__ __launch_bounds__(256) void k_world(WorldArgs W)
 // It also zeroes the tile counts and fill ranks and the counter words
 // [w0, w0 + n_words) that the binning kernels after it accumulate into, and
 // marks every tile as without an offset.
-__global__ __launch_bounds__(256) void k_vertex(BatchDev B, uint32_t w0, uint32_t n_words, const JobDev *__restrict__ jobs)
+__device__ __forceinline__ void vertex_block(const BatchDev &B, uint32_t w0, uint32_t n_words, const JobDev &J)
 {
     const uint32_t gi = blockIdx.x * 256u + threadIdx.x, stride = gridDim.x * 256u;
     for (uint32_t k = gi; k < B.n_tiles; k += stride) {
@@ -149,7 +149,6 @@ __global__ __launch_bounds__(256) void k_vertex(BatchDev B, uint32_t w0, uint32_
     }
     for (uint32_t k = gi; k < n_words; k += stride)
         B.ctr[w0 + k] = 0;
-    const JobDev &J = jobs[find_job<JV>(B, jobs, blockIdx.x)];
     const uint32_t i = (blockIdx.x - J.vblock0) * 256u + threadIdx.x;
     if (i >= J.n_vertices)
         return;
@@ -159,6 +158,21 @@ __global__ __launch_bounds__(256) void k_vertex(BatchDev B, uint32_t w0, uint32_
     // every setup of a triangle with this vertex would divide out again
     J.ndc[i] = make_float4(f.x, f.y, f.z, 1.0f / f.z);
     J.yes[i] = 0;
+}
+__global__ __launch_bounds__(256) void k_vertex(BatchDev B, uint32_t w0, uint32_t n_words, const JobDev *__restrict__ jobs)
+{
+    vertex_block(B, w0, n_words, jobs[find_job<JV>(B, jobs, blockIdx.x)]);
+}
+// The same for a wave of one job, whose table arrives with the arguments (488
+// bytes) and is left in memory for the kernels after it: a copy of its own
+// ahead of the kernels is one more operation on the stream that every frame
+// waits for (640x480 cube 39 us a frame with it, 35 without; 800x600 demo
+// scene 57 and 50; 1280x720 field posed anew 119 and 114).
+__global__ __launch_bounds__(256) void k_vertex_one(BatchDev B, uint32_t w0, uint32_t n_words, JobDev J)
+{
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        *const_cast<JobDev *>(B.jobs) = J;
+    vertex_block(B, w0, n_words, J);
 }
 
 // A triangle's three vertices carry visibility marks (renderer.cpp:248-253
@@ -2690,9 +2704,14 @@ hipError_t launch_world(const WorldArgs &W, hipStream_t s)
         LAUNCH_CHECK(k_world, dim3((W.n_vertices + 255) / 256), dim3(256), 0, s, W);
     return hipSuccess;
 }
-hipError_t launch_vertex(const BatchDev &B, uint32_t blocks, uint32_t w0, uint32_t n_words, hipStream_t s)
+hipError_t launch_vertex(const BatchDev &B, uint32_t blocks, uint32_t w0, uint32_t n_words, const JobDev *one,
+                         hipStream_t s)
 {
     // at least one block: the kernel also zeroes the counters
+    if (one) {
+        LAUNCH_CHECK(k_vertex_one, dim3(blocks ? blocks : 1), dim3(256), 0, s, B, w0, n_words, *one);
+        return hipSuccess;
+    }
     LAUNCH_CHECK(k_vertex, dim3(blocks ? blocks : 1), dim3(256), 0, s, B, w0, n_words, B.jobs);
     return hipSuccess;
 }
@@ -2784,7 +2803,7 @@ hipError_t launch_dof(const BatchDev &B, uint32_t blocks, int max_radius, hipStr
 hipError_t resolve_kernels()
 {
     const void *k[] = {
-        (const void *)k_world, (const void *)k_vertex, (const void *)k_front, (const void *)k_bin_fill,
+        (const void *)k_world, (const void *)k_vertex, (const void *)k_vertex_one, (const void *)k_front, (const void *)k_bin_fill,
         (const void *)k_raster<8, 8, false>, (const void *)k_raster<16, 16, false>,
         (const void *)k_raster<32, 16, false>, (const void *)k_raster<32, 32, false>,
         (const void *)k_raster<64, 32, false>, (const void *)k_raster<64, 64, false>,

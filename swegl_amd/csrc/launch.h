@@ -5,7 +5,9 @@
 
 namespace sw {
 hipError_t launch_world(const WorldArgs &W, hipStream_t s);
-hipError_t launch_vertex(const BatchDev &B, uint32_t blocks, uint32_t w0, uint32_t n_words, hipStream_t s);
+// `one`: the table of a wave of one job, on the host; null: already at B.jobs
+hipError_t launch_vertex(const BatchDev &B, uint32_t blocks, uint32_t w0, uint32_t n_words, const JobDev *one,
+                         hipStream_t s);
 // marks, tile rectangles and counts, and (last block) the scan into bin offsets
 hipError_t launch_front(const BatchDev &B, uint32_t blocks, hipStream_t s);
 // the fill over `blocks` blocks, plus the blocks that write the claim order;
