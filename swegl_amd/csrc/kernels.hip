@@ -1606,12 +1606,15 @@ __device__ __forceinline__ uint32_t raster_tile(const BatchDev &B, const JobDev 
                 const uint32_t kn2 = ro(bins)[min(e + 2u * NT, nb - 1u)];
                 const bool drawn = !(k & flags & SW_BIN_CHECK) ||
                                    ((ro(W.yes)[i0] != 0) & (ro(W.yes)[i1] != 0) & (ro(W.yes)[i2] != 0));
-                // (in a band most entries lie in other rows)
-                const bool here = !band || !(fmaxf(T.a.y, fmaxf(T.b.y, T.c.y)) <= (float)W.tr.y0 ||
-                                             fminf(T.a.y, fminf(T.b.y, T.c.y)) > (float)(W.tr.y1 - 1));
+                // In a band most entries lie in other rows, which only a plain
+                // triangle's vertices tell: a near-clipped one also covers
+                // rows beyond its projected vertices.
+                const bool plain = is_plain(T);
+                const bool here = !band || !plain || !(fmaxf(T.a.y, fmaxf(T.b.y, T.c.y)) <= (float)W.tr.y0 ||
+                                                       fminf(T.a.y, fminf(T.b.y, T.c.y)) > (float)(W.tr.y1 - 1));
                 if (drawn && here) {
                     int ry0, ry1;
-                    if (!is_plain(T) ||
+                    if (!plain ||
                         ((k & flags & SW_BIN_LARGE) && rows_of(T, true, ry0, ry1) > SW_LANE_PIXELS))
                         list(t);
                     else
