@@ -1567,14 +1567,17 @@ __device__ __forceinline__ uint32_t raster_tile(const BatchDev &B, const JobDev 
         return max(ry1 - ry0, 0) * w;
     };
     // Entry e of the tile: its triangle, whether its marks are still to be
-    // looked up and whether it may cover many pixels (neither is ever set in
-    // the filled layout); false: a big triangle elsewhere.
+    // looked up and whether it may cover many pixels (the filled layout holds
+    // marked triangles and does not tell their sizes: there every triangle's
+    // pixels are counted, without which a lane replays a large one alone,
+    // 8,000 small triangles and 8 large ones in a 320x320 view 87 us by
+    // swegl_render_noalloc, 67 with it); false: a big triangle elsewhere.
     auto entry = [&](uint32_t e, uint32_t &t, bool &check, bool &large) -> bool {
         if (e < nb) {
             const uint32_t k = ro(bins)[e], flags = fixed ? k & (SW_BIN_CHECK | SW_BIN_LARGE) : 0u;
             t = k ^ flags;
             check = (flags & SW_BIN_CHECK) != 0;
-            large = (flags & SW_BIN_LARGE) != 0;
+            large = !fixed || (flags & SW_BIN_LARGE) != 0;
             return true;
         }
         const JobDev &B1 = reread(jobs, jidx);
@@ -1624,7 +1627,7 @@ __device__ __forceinline__ uint32_t raster_tile(const BatchDev &B, const JobDev 
                 if (drawn && here) {
                     int ry0, ry1;
                     if (!plain ||
-                        ((k & flags & SW_BIN_LARGE) && rows_of(T, true, ry0, ry1) > SW_LANE_PIXELS))
+                        ((!fixed || (k & SW_BIN_LARGE)) && rows_of(T, true, ry0, ry1) > SW_LANE_PIXELS))
                         list(t);
                     else
                         plain_depth<TW, SLOTS>(W, T, t, i0, i1, i2, W.tr.y0, W.tr.y1, W.tr.x0, W.tr.x1, keys, slots, NSLOT,
