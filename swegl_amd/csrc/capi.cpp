@@ -819,27 +819,9 @@ extern "C" int swegl_scene_upload(swegl_ctx *c, const swegl_scene_desc *d, swegl
         return fail(SWEGL_EINVAL, "null argument");
     HIPCHK(hipSetDevice(c->device));
     std::unique_ptr<swegl_scene> s(new swegl_scene);
-    // ---- validate and flatten primitives in draw order (nodes, then primitives)
-    // the arrays' sizes first (what is out of range is refused below)
+    // ---- the whole description is checked, and what it holds counted, before
+    // anything is allocated or filled
     uint64_t nv = 0, nt = 0;
-    for (uint32_t ni = 0; ni < d->n_nodes; ni++) {
-        const swegl_node_desc &nd = d->nodes[ni];
-        if ((uint64_t)nd.first_primitive + nd.n_primitives > d->n_primitives)
-            break;
-        for (uint32_t k = 0; k < nd.n_primitives; k++) {
-            const swegl_primitive_desc &p = d->primitives[nd.first_primitive + k];
-            nv += p.n_vertices;
-            if (p.mode == SWEGL_TRIANGLES)
-                nt += p.n_indices / 3;
-            else if ((p.mode == SWEGL_TRIANGLE_STRIP || p.mode == SWEGL_TRIANGLE_FAN) && p.n_indices >= 3)
-                nt += p.n_indices - 2;
-        }
-    }
-    if (nv > 0x7FFFFFFFu || nt > 0x7FFFFFFFu)
-        return fail(SWEGL_EINVAL, "scene too large");
-    std::vector<float> px(nv), py(nv), pz(nv), nx(nv), ny(nv), nz(nv), tu(nv), tv(nv);
-    std::vector<uint32_t> tri(4 * nt);
-    size_t v_at = 0, t_at = 0;   // vertices and words of `tri` written
     for (uint32_t ni = 0; ni < d->n_nodes; ni++) {
         const swegl_node_desc &nd = d->nodes[ni];
         if ((uint64_t)nd.first_primitive + nd.n_primitives > d->n_primitives)
@@ -855,17 +837,42 @@ extern "C" int swegl_scene_upload(swegl_ctx *c, const swegl_scene_desc *d, swegl
             // such a scene (swegl_scene::no_material)
             if (p.material_id < -1 || p.material_id >= (int)d->n_materials)
                 return fail(SWEGL_EINVAL, "material_id %d out of range", p.material_id);
-            const bool nomat = p.material_id == -1;
-            const swegl_material_desc &m = nomat ? d->default_material : d->materials[p.material_id];
-            if (!nomat && (m.texture_idx < -1 || m.texture_idx >= (int)d->n_textures))
-                return fail(SWEGL_EINVAL, "texture_idx %d out of range", m.texture_idx);
-            s->no_material = s->no_material || nomat;
+            if (p.material_id != -1) {
+                const int32_t tex = d->materials[p.material_id].texture_idx;
+                if (tex < -1 || tex >= (int)d->n_textures)
+                    return fail(SWEGL_EINVAL, "texture_idx %d out of range", tex);
+            }
             if (p.n_vertices && (!p.positions || !p.normals || !p.tex_coords))
                 return fail(SWEGL_EINVAL, "null vertex arrays");
             for (uint32_t i = 0; i < p.n_indices; i++)
                 if (p.indices[i] >= p.n_vertices)
                     return fail(SWEGL_EINVAL, "index %u out of range (%u vertices)", p.indices[i],
                                 p.n_vertices);
+            nv += p.n_vertices;
+            if (p.mode == SWEGL_TRIANGLES)
+                nt += p.n_indices / 3;
+            else if ((p.mode == SWEGL_TRIANGLE_STRIP || p.mode == SWEGL_TRIANGLE_FAN) && p.n_indices >= 3)
+                nt += p.n_indices - 2;
+        }
+    }
+    if (nv > 0x7FFFFFFFu || nt > 0x7FFFFFFFu)
+        return fail(SWEGL_EINVAL, "scene too large");
+    for (uint32_t i = 0; i < d->n_textures; i++) {
+        const swegl_texture_desc &t = d->textures[i];
+        if (!t.bitmap || t.width == 0 || t.height == 0 || t.width > 65536 || t.height > 65536)
+            return fail(SWEGL_EINVAL, "texture %u is empty or too large", i);
+    }
+    // ---- flatten primitives in draw order (nodes, then primitives)
+    std::vector<float> px(nv), py(nv), pz(nv), nx(nv), ny(nv), nz(nv), tu(nv), tv(nv);
+    std::vector<uint32_t> tri(4 * nt);
+    size_t v_at = 0, t_at = 0;   // vertices and words of `tri` written
+    for (uint32_t ni = 0; ni < d->n_nodes; ni++) {
+        const swegl_node_desc &nd = d->nodes[ni];
+        for (uint32_t k = 0; k < nd.n_primitives; k++) {
+            const swegl_primitive_desc &p = d->primitives[nd.first_primitive + k];
+            const bool nomat = p.material_id == -1;
+            const swegl_material_desc &m = nomat ? d->default_material : d->materials[p.material_id];
+            s->no_material = s->no_material || nomat;
             PrimDev pd;
             pd.first_vertex = (uint32_t)v_at;
             pd.n_vertices = p.n_vertices;
@@ -917,11 +924,8 @@ extern "C" int swegl_scene_upload(swegl_ctx *c, const swegl_scene_desc *d, swegl
     std::vector<uint64_t> first_texel(d->n_textures);
     uint64_t texels = 0;
     for (uint32_t i = 0; i < d->n_textures; i++) {
-        const swegl_texture_desc &t = d->textures[i];
-        if (!t.bitmap || t.width == 0 || t.height == 0 || t.width > 65536 || t.height > 65536)
-            return fail(SWEGL_EINVAL, "texture %u is empty or too large", i);
         first_texel[i] = texels;
-        texels += (uint64_t)t.width * t.height;
+        texels += (uint64_t)d->textures[i].width * d->textures[i].height;
     }
     for (PrimDev &pd : s->h_prims) {
         pd.texel = pd.tex >= 0 ? first_texel[pd.tex] : 0;
