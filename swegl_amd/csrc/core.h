@@ -79,10 +79,12 @@ SW_HD float dot(f3 a, f3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
 //    all 1.6e9 of them);
 //  - div_rn: with r = rcp_rn(b), one residual correction equals a / b for
 //    every pair of significands (all 2^46 compared on the device through the
-//    exact residual) while a and the quotient stay within 2^-90 .. 2^120 and
-//    b within 2^-47 .. 2^47 (the residual is then exact); a positive zero a
-//    gives a positive zero.
-// A GPU test repeats the unary comparisons in full and samples the quotients.
+//    exact residual) while a stays within 2^-102 .. 2^120, the quotient
+//    within 2^-90 .. 2^120 and b within 2^-47 .. 2^47: the residual is then
+//    exact, as a whole multiple of 2^-149 (denormals are kept); a positive
+//    zero a gives a positive zero.  The lights' second quotient has the
+//    smallest numerators (shade.h).
+// GPU tests repeat the unary comparisons in full and sample the quotients.
 SW_D float rcp_rn(float b)
 {
     const float r0 = __builtin_amdgcn_rcpf(b);
