@@ -4,8 +4,8 @@
 // same float operations in the same order (the library is compiled with
 // -ffp-contract=off; HIP's default IEEE division and square root).  The
 // x86-64 conversion semantics of the reference build (cvttss2si: NaN and
-// out-of-range -> INT32_MIN, float -> uint8 through a 32-bit int) are
-// emulated explicitly because v_cvt_i32_f32 saturates instead.
+// out-of-range -> INT32_MIN) are emulated explicitly where a value may be out
+// of range, because v_cvt_i32_f32 saturates instead.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -47,7 +47,6 @@ SW_HD int32_t cvtt(float f)
 {
     return (f >= -2147483648.0f && f < 2147483648.0f) ? (int32_t)f : INT32_MIN;
 }
-SW_HD uint8_t to_u8(float f) { return (uint8_t)(uint32_t)cvtt(f); }
 SW_HD int32_t wrap_add(int32_t a, int32_t b) { return (int32_t)((uint32_t)a + (uint32_t)b); }
 
 // `z <= 0.001` with z a float and 0.001 a double literal (renderer.cpp:489)

@@ -888,7 +888,7 @@ struct TileRect { int x0, y0, x1, y1; };   // [x0,x1) x [y0,y1), absolute pixels
 // by a fragment it beat carries another tag.  So where all three tags name
 // the final winner, the payload is the winner's own, and the shading needs
 // no replay of its setup, rows or span; elsewhere (a race, a sequence of
-// 2^30 or more) the pixel is shaded the long way.
+// 2^25 or more: triangles from 2^24 on) the pixel is shaded the long way.
 // Tag: the sequence (25 bits), then the sub-triangle's vertex order in
 // fill_triangle_2 as (index of S.v[0], of S.v[1]) among the triangle's
 // three vertices, 3 * p0 + p1 (15: a clip vertex is among them), whether it
@@ -2134,7 +2134,7 @@ __device__ __forceinline__ uint32_t blend_colors(uint32_t back, uint32_t front)
 
 // The fragments of triangle t's unclipped sub-triangle over the tile's rows
 // [row0, row1) and columns [tx0, tx0 + TW): the same row walk and span
-// stepping as raster_depth (renderer.cpp:462-558), writing each covered
+// stepping as raster_depth_any (renderer.cpp:462-558), writing each covered
 // pixel's depth to z[py * TW + px] and its bit to the returned mask.  With
 // `opaque`, also the bit of every covered pixel whose texture-part colour
 // (frag_texture: material colour, nearest or bilinear texel) has alpha 255,
