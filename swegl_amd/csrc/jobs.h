@@ -171,9 +171,11 @@ struct BatchDev {
 #define SW_TICKET_GROUPS 32
 #define SW_CTR_OVERFLOW (SW_CTR_TOTAL + 32)   // tiles that passed tile_cap
 // Each raster queue's number of items, then of empty tiles after them; the
-// claims of those (a line of its own for each queue)
+// claims of those of queue k at SW_CTR_EMPTYQ + 64k, on the second 128-byte
+// line beside its counter (what swegl_render_noalloc's array holds and a
+// server's budget admits hangs on the block's size)
 #define SW_CTR_ITEMS (SW_CTR_TOTAL + 34)
-#define SW_CTR_EMPTYQ (SW_CTR_TOTAL + 64)
+#define SW_CTR_EMPTYQ (SW_CTR_QUEUE0 + 32)
 // A fixed-layout bin entry with this bit set names a triangle that failed its
 // own visibility test: it is drawn only if other triangles marked all three
 // of its vertices, which the raster looks up
@@ -181,7 +183,7 @@ struct BatchDev {
 // and one with this bit set a triangle whose bounding box holds more than
 // SW_LANE_PIXELS pixels (a job of the fixed layout holds < 2^30 triangles)
 #define SW_BIN_LARGE 0x40000000u
-#define SW_CTR_TICKETS (SW_CTR_EMPTYQ + 32 * SW_RASTER_QUEUES)
+#define SW_CTR_TICKETS (SW_CTR_TOTAL + 64)
 #define SW_CTR_BIG0 (SW_CTR_TICKETS + 32 * (SW_TICKET_GROUPS + 1))
 // statistic indices within a slot
 #define SW_ST_FRAGMENTS 0

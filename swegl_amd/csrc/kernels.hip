@@ -1968,7 +1968,7 @@ k_raster(BatchDev B, const JobDev *__restrict__ jobs)
         while (E) {
             __syncthreads();
             if (threadIdx.x == 0)
-                s_place = atomicAdd(B.ctr + SW_CTR_EMPTYQ + 32 * k, (uint32_t)SW_EMPTY_CLAIM);
+                s_place = atomicAdd(B.ctr + SW_CTR_EMPTYQ + 64 * k, (uint32_t)SW_EMPTY_CLAIM);
             __syncthreads();
             uint32_t c = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_place);
             if (c >= E)
